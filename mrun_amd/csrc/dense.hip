@@ -76,7 +76,8 @@ __global__ __launch_bounds__(256 * KG) void dense_gemm_kernel(DenseJob j) {
                 const int i = i0 + u * step;
                 if (i >= DBM * bpr) break;  // uniform: the same count for every thread
                 const int row = r0 + i / bpr, blk = kq * bpr + i % bpr;
-                pack_block_v(v[u], min(row, j.M - 1), row < j.M, j.K, blk, j.pack_a, j.K, j.pack_x);
+                pack_block_v(v[u], min(row, j.M - 1), row < j.M, j.K, blk, j.pack_a, j.K, j.pack_x,
+                             j.pack_g);
             }
         }
         return;

@@ -191,20 +191,21 @@ constexpr int kGemmTileM = 64;  // rows per routed tile
 
 constexpr int kGemmTileN = 64;
 
-// The prefill forward's grouped expert GEMM (moe_gemm.hip): 4-bit group-64 weights (biases may be
-// null), K % 512 == 0, N a multiple of 128 (glu) or 256. A is packed (launch_apack) with its X
-// splits AX [rows][3][ax_e] (ax_e = K / 64: one entry per group).
+// The prefill forward's grouped expert GEMM (4-bit group-64 weights: moe_gemm.hip; 4-bit groups of
+// 32 or 128, 8-bit and bf16 weights: moe_fmt.hip; biases may be null), K % 512 == 0, N a multiple
+// of 128 (glu) or 256. A is packed (launch_apack) with its X splits AX [rows][3][ax_e] (one entry
+// per ax_g inputs: 32 for weights in groups of 32, else 64; bf16 weights read none).
 // Routed tiles come from routing.tiles (64 rows); their A rows from tile_rows [tile][64] (token
 // of each tile row; only the tile's rows are read, rows past them repeat its last one) or,
-// without tile_rows, the sorted positions themselves. glu: out = packed R(silu(R(A.w0)) * R(A.w1)) and OX [rows][3][N / 64]
-// the X splits of each output row's groups; else out = R(A.w0). The shared product (sh)
+// without tile_rows, the sorted positions themselves. glu: out = packed R(silu(R(A.w0)) * R(A.w1)) and OX
+// [rows][3][N / ox_g] the X splits of each output row's groups of ox_g (0: none); else out = R(A.w0). The shared product (sh)
 // has the same K and N and comes first.
 struct MoeGemmJob {
     const bf16_t *A;
     int lda;
     int a_rows;  // rows of A (its byte offsets are 32-bit: a_rows * lda * 2 < 2^32)
     const bf16_t *AX;
-    int ax_e;
+    int ax_e, ax_g;
     const uint32_t *tile_rows;
     int K, N, glu;
     QW w0, w1;
@@ -215,6 +216,7 @@ struct MoeGemmJob {
     bf16_t *out;
     int ldo;
     bf16_t *OX;
+    int ox_g;
     struct {
         const bf16_t *A;
         int lda;
@@ -230,9 +232,13 @@ struct MoeGemmJob {
 };
 bool moe_gemm_supported(const MoeGemmJob &j);
 hipError_t launch_moe_gemm(const MoeGemmJob &j, hipStream_t stream);
-// x [rows][K] (row stride lda) -> packed rows (stride ldp) and X splits [rows][3][K / 64]
+// moe_fmt.hip's part of the two above (the checks that depend on the weights' format)
+bool fmt_gemm_supported(const MoeGemmJob &j);
+hipError_t launch_fmt_gemm(const MoeGemmJob &j, unsigned grid, hipStream_t stream);
+// x [rows][K] (row stride lda) -> packed rows (stride ldp) and X splits [rows][3][K / xg], xg 32
+// or 64
 hipError_t launch_apack(const bf16_t *x, int lda, int rows, int K, bf16_t *xp, int ldp,
-                        bf16_t *xs, hipStream_t stream);
+                        bf16_t *xs, int xg, hipStream_t stream);
 
 // Dense bf16 Linear for more than 16 rows on the MFMAs (dense.hip): out0 = R(A W0^T) then
 // R(. + bias0), and optionally out1 from W1 in the same launch (the shared expert's gate beside the
@@ -251,8 +257,9 @@ struct DenseJob {
     uint32_t *zero;
     int n_zero;
     // optional: A packed for the grouped GEMM (launch_apack's layout and bits: pack_a [M][K],
-    // pack_x [M][3][K / 64]) by extra workgroups of the same launch
+    // pack_x [M][3][K / pack_g]) by extra workgroups of the same launch
     bf16_t *pack_a, *pack_x;
+    int pack_g;
 };
 bool dense_gemm_supported(int M, int K);
 hipError_t launch_dense_gemm(const DenseJob &job, hipStream_t stream);

@@ -176,6 +176,7 @@ struct Plan {
     size_t counts;
     int n_counts;
     size_t xp, xs, act_x, sh_act_x, tile_rows;  // the packed operands of the prefill GEMMs
+    bool x32;  // xs, act_x and sh_act_x hold X sums of 32 inputs (else of 64)
     size_t act, y, sh_logit, sh_act, sh_y, total;
     int max_tiles;
 };
@@ -217,12 +218,29 @@ static Plan make_plan(const mrun_moe_config &c, int T) {
         p.sh_y = take(2 * (size_t)T * D);
     }
     // prefill GEMM operands (moe_gemm.hip): packed x and its group-sum splits, the group-sum
-    // splits of act (and of the shared expert's act), the token rows of each routed tile
+    // splits of act (and of the shared expert's act), the token rows of each routed tile. Weights in
+    // groups of 32 take twice the sums. The plan has room for them where packed x fits in y (x is
+    // packed before the gate/up launch, its last reader; y is written by the down launch), as long
+    // as that needs no more than a plan with packed x of its own and sums of 64: a fixed scratch
+    // then holds as many tokens as without them.
     if (T > 16) {
-        p.xp = take(2 * (size_t)T * D);
-        p.xs = take(2 * 3 * (size_t)T * (D / 64));
-        p.act_x = take(2 * 3 * P * (I / 64));
-        if (S > 0) p.sh_act_x = take(2 * 3 * (size_t)T * (S / 64));
+        auto sums = [&](size_t n, size_t xg) { return 2 * 3 * n * xg; };
+        const size_t xp = a256(2 * (size_t)T * D), y = a256(2 * P * D);
+        auto need = [&](size_t g) {
+            return a256(sums(P, I / g)) + (S > 0 ? a256(sums(T, S / g)) : 0);
+        };
+        const size_t own = xp + a256(sums(T, D / 64)) + need(64);
+        p.x32 = xp + a256(sums(T, D / 32)) <= y && need(32) <= own;
+        if (p.x32) {
+            p.xp = p.y;
+            p.xs = p.y + xp;
+        } else {
+            p.xp = take(2 * (size_t)T * D);
+            p.xs = take(sums(T, D / 64));
+        }
+        const size_t g = p.x32 ? 32 : 64;
+        p.act_x = take(sums(P, I / g));
+        if (S > 0) p.sh_act_x = take(sums(T, S / g));
         p.tile_rows = take(4 * (size_t)p.max_tiles * kGemmTileM);
     }
     p.total = at;
@@ -506,6 +524,10 @@ static Status sparse_moe_forward(const mrun_sparse_moe &m, const bf16_t *x, int 
     // by its own launch after the routing
     const bool packs = mfma && T > 16 && D % 512 == 0 && I % 512 == 0;
     bool packed = false;
+    // inputs per X sum of x and of act: the group of the weights they meet, at most 64
+    auto x_group = [](const mrun_quantized &q) { return q.bits != 16 && q.group_size == 32 ? 32 : 64; };
+    const int xg = x_group(m.switch_gate_proj), og = x_group(m.switch_down_proj);
+    const bool x_fits = p.x32 || (xg == 64 && og == 64);
     if (m.gate.weight && (!S || m.shared_expert_gate.weight) && dense_gemm_supported(T, D)) {
         // router and shared gate: one launch over x
         DenseJob dj{};
@@ -516,7 +538,10 @@ static Status sparse_moe_forward(const mrun_sparse_moe &m, const bf16_t *x, int 
             dj.N1 = 1, dj.out1 = sh_logit, dj.ldo1 = 1;
         }
         dj.zero = counts, dj.n_zero = p.n_counts;
-        if (packs) dj.pack_a = (bf16_t *)at(p.xp), dj.pack_x = (bf16_t *)at(p.xs), packed = true;
+        if (packs && x_fits) {
+            dj.pack_a = (bf16_t *)at(p.xp), dj.pack_x = (bf16_t *)at(p.xs), dj.pack_g = xg;
+            packed = true;
+        }
         TRY_HIP(launch_dense_gemm(dj, s), "router (mfma)");
         st.mark(s);  // (the shared gate's stage below stays empty: it ran in this launch)
     } else {
@@ -528,45 +553,49 @@ static Status sparse_moe_forward(const mrun_sparse_moe &m, const bf16_t *x, int 
     TRY_HIP(launch_topk_count(logits, T, E, k, c.norm_topk_prob != 0, ids, scores, counts, s),
             "top-k");
     st.mark(s);
-    // the grouped GEMM of moe_gemm.hip: 4-bit group-64 experts, K a multiple of 512, the shared
-    // expert in the same launches when its width equals the routed one
+    // mid-size batches: the routed tiles cut to 32 rows (most experts hold a few rows, so a 64-row
+    // tile is mostly padding), on the grouped GEMM's one-row-fragment instantiation; bf16 experts
+    // run 32-row tiles at every size
+    const bool half = (long long)P <= (long long)kHalfTileMaxRows * E ||
+                      m.switch_gate_proj.bits == 16 || m.switch_down_proj.bits == 16;
+    // the grouped GEMM (moe_gemm.hip, moe_fmt.hip): K a multiple of 512, the shared expert in the
+    // same launches when its width and format equal the routed ones
     MoeGemmJob mg{}, md{};
     bool new_path = false, fuse_new = false;
-    if (mfma && T > 16) {
+    if (packs && x_fits) {
+        mg.tile_m = md.tile_m = half ? 32 : kGemmTileM;
         mg.A = (const bf16_t *)at(p.xp), mg.lda = D, mg.a_rows = T, mg.AX = (const bf16_t *)at(p.xs);
-        mg.ax_e = D / 64, mg.tile_rows = (const uint32_t *)at(p.tile_rows);
+        mg.ax_g = xg, mg.ax_e = D / xg, mg.tile_rows = (const uint32_t *)at(p.tile_rows);
         mg.K = D, mg.N = I, mg.glu = 1;
         mg.w0 = qw_of(m.switch_gate_proj), mg.w1 = qw_of(m.switch_up_proj);
         mg.routing = rt, mg.has_routing = 1, mg.max_tiles = p.max_tiles;
+        // bf16 down weights read no sums (the 4-bit group-64 kernel writes them all the same)
         mg.out = act, mg.ldo = I, mg.OX = (bf16_t *)at(p.act_x);
-        md.A = act, md.lda = I, md.a_rows = P, md.AX = (const bf16_t *)at(p.act_x), md.ax_e = I / 64;
+        mg.ox_g = m.switch_gate_proj.bits == 16 && m.switch_down_proj.bits == 16 ? 0 : og;
+        md.A = act, md.lda = I, md.a_rows = P, md.AX = (const bf16_t *)at(p.act_x);
+        md.ax_g = og, md.ax_e = I / og;
         md.K = I, md.N = D, md.glu = 0, md.w0 = qw_of(m.switch_down_proj);
         md.routing = rt, md.has_routing = 1, md.max_tiles = p.max_tiles, md.out = y, md.ldo = D;
         new_path = moe_gemm_supported(mg) && moe_gemm_supported(md);
-        if (new_path && S == I && !m.shared_gate_proj.weight && !m.shared_up_proj.weight &&
-            !m.shared_down_proj.weight) {
+        if (new_path && S == I) {
             MoeGemmJob tg = mg, td = md;
-            tg.sh = {mg.A, D, mg.AX, D / 64, T, qw_of(m.shared_gate_proj.q),
-                     qw_of(m.shared_up_proj.q), sh_act, S, (bf16_t *)at(p.sh_act_x)};
+            tg.sh = {mg.A, D, mg.AX, mg.ax_e, T, qw_of(as_quantized(m.shared_gate_proj)),
+                     qw_of(as_quantized(m.shared_up_proj)), sh_act, S, (bf16_t *)at(p.sh_act_x)};
             tg.has_shared = 1;
-            td.sh = {sh_act, S, (const bf16_t *)at(p.sh_act_x), S / 64, T,
-                     qw_of(m.shared_down_proj.q), QW{}, sh_y, D, nullptr};
+            td.sh = {sh_act, S, (const bf16_t *)at(p.sh_act_x), md.ax_e, T,
+                     qw_of(as_quantized(m.shared_down_proj)), QW{}, sh_y, D, nullptr};
             td.has_shared = 1;
             if (moe_gemm_supported(tg) && moe_gemm_supported(td)) mg = tg, md = td, fuse_new = true;
         }
     }
-    // mid-size batches: the routed tiles cut to 32 rows (most experts hold a few rows, so a 64-row
-    // tile is mostly padding), on the grouped GEMM's one-row-fragment instantiation
-    const bool half = new_path && (long long)P <= (long long)kHalfTileMaxRows * E;
-    mg.tile_m = md.tile_m = half ? 32 : kGemmTileM;
     PermuteOut pt = po;
-    pt.tile_m = half ? 32 : kGemmTileM;
+    pt.tile_m = new_path && half ? 32 : kGemmTileM;
     pt.tiles = (uint32_t *)at(p.tiles);
     pt.n_tiles = (uint32_t *)at(p.n_tiles);
-    if (packs) pt.tile_rows = (uint32_t *)at(p.tile_rows);
+    if (new_path) pt.tile_rows = (uint32_t *)at(p.tile_rows);
     TRY_HIP(launch_route_scatter(ids, counts, T, k, E, pt, s), "scatter");
-    if (packs && !packed)
-        TRY_HIP(launch_apack(x, D, T, D, (bf16_t *)at(p.xp), D, (bf16_t *)at(p.xs), s), "pack x");
+    if (new_path && !packed)
+        TRY_HIP(launch_apack(x, D, T, D, (bf16_t *)at(p.xp), D, (bf16_t *)at(p.xs), xg, s), "pack x");
     st.mark(s);
     if (new_path) {
         TRY_HIP(launch_moe_gemm(mg, s), "gate/up (moe gemm)");
@@ -1123,7 +1152,7 @@ int mrun_gather_qmm(const mrun_bf16 *x, int32_t x_rows, const mrun_quantized *w,
         if (n > 16) {
             mj.A = (const bf16_t *)(ws + p.xp), mj.lda = w->in, mj.a_rows = x_rows;
             mj.AX = (const bf16_t *)(ws + p.xs);
-            mj.ax_e = w->in / 64, mj.tile_rows = u32(p.tile_rows), mj.K = w->in, mj.N = w->out;
+            mj.ax_g = 64, mj.ax_e = w->in / 64, mj.tile_rows = u32(p.tile_rows), mj.K = w->in, mj.N = w->out;
             mj.glu = 0, mj.w0 = qw_of(*w), mj.routing = rt, mj.has_routing = 1;
             mj.max_tiles = (int)p.max_tiles, mj.out = (bf16_t *)(ws + p.ys), mj.ldo = w->out;
         }
@@ -1133,7 +1162,7 @@ int mrun_gather_qmm(const mrun_bf16 *x, int32_t x_rows, const mrun_quantized *w,
                         "gather_qmm permute");
         if (st.ok() && tuned) {
             st = hip_status(launch_apack(x, w->in, x_rows, w->in, (bf16_t *)(ws + p.xp), w->in,
-                                         (bf16_t *)(ws + p.xs), s),
+                                         (bf16_t *)(ws + p.xs), 64, s),
                             "gather_qmm pack x");
             if (st.ok()) st = hip_status(launch_moe_gemm(mj, s), "gather_qmm (moe gemm)");
             if (st.ok())
