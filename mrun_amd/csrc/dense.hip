@@ -14,6 +14,15 @@
 // across it. A step issues its MFMAs first and then stages the next step's tile, so the matrix
 // cores run while the stores and the barrier wait.
 //
+// Q8: an 8-bit router and shared gate (mlx-community conversions), groups of 64 or 128. The codes
+// become exact bf16 integers when a tile is staged; each K step's MFMA chain starts from zero and
+// enters the result as  s * P + b * X  with X the step's sum of x, so no weight is rounded. The
+// launch reads half the dense router's bytes, and waits on the same latency: at 1000 tokens of the
+// Qwen3.6-like block the router, gate and packing took 48 us as four launches of the register-staged
+// GEMM of qgemm.hip (26 + 12), a fill (5) and the packing (5); one launch of this kernel took 32 us
+// off that block (313 -> 281 us per forward, 303 -> 269 at 2048 tokens of 4-bit experts, 158 -> 123
+// at 50).
+//
 // With pack_a set, extra workgroups of the launch (column blocks past the product's, one per row
 // block and quarter of K) write A in the grouped GEMM's packed layout with launch_apack's code, bit
 // for bit. They run beside the product on the CUs it leaves idle; folded into the product's own
@@ -38,9 +47,21 @@ constexpr int DBM = 64, DBN = 64, DBK = 64, DLDK = DBK + 8;
 
 struct Stage {
     uint4 a0, a1, b0, b1;
+    uint32_t sb;  // Q8: the row's scale (low half) and bias of this K step, b0 its 16 codes
 };
 
-template <int NST, int KG>
+// four 8-bit codes -> bf16 pairs (q0, q1), (q2, q3): integers below 256 are exact in bf16, so the
+// top half of their f32 conversion is their bf16
+__device__ __forceinline__ uint2 q8_pairs(uint32_t w) {
+    const uint32_t f0 = __float_as_uint((float)(w & 0xffu));
+    const uint32_t f1 = __float_as_uint((float)((w >> 8) & 0xffu));
+    const uint32_t f2 = __float_as_uint((float)((w >> 16) & 0xffu));
+    const uint32_t f3 = __float_as_uint((float)(w >> 24));
+    return make_uint2(__builtin_amdgcn_perm(f1, f0, 0x07060302u),
+                      __builtin_amdgcn_perm(f3, f2, 0x07060302u));
+}
+
+template <int NST, int KG, bool Q8>
 __global__ __launch_bounds__(256 * KG) void dense_gemm_kernel(DenseJob j) {
     // per group: A and B tiles, double-buffered; after the K loop the first KG - 1 groups' 4 x 64
     // x 16 partial sums reuse the space (KG - 1 groups x 16 KB <= KG x 36 KB)
@@ -48,12 +69,13 @@ __global__ __launch_bounds__(256 * KG) void dense_gemm_kernel(DenseJob j) {
     const int kg = threadIdx.x >> 8, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
     bf16_t(*As)[DBM * DLDK] = stage_lds[kg][0];
     bf16_t(*Bs)[DBN * DLDK] = stage_lds[kg][1];
+    __shared__ __align__(16) float q8_lds[Q8 ? KG : 1][2][3][Q8 ? DBM : 4];  // X, scales, biases
     if (j.zero && blockIdx.x == 0 && blockIdx.y == 0)
         for (int i = threadIdx.x; i < j.n_zero; i += 256 * KG) j.zero[i] = 0;
 
     // column block -> weight (W0's blocks first, then W1's, then the packing blocks)
     const int nb0 = (j.N0 + DBN - 1) / DBN;
-    const int nbw = nb0 + (j.W1 ? (j.N1 + DBN - 1) / DBN : 0);
+    const int nbw = nb0 + (j.N1 ? (j.N1 + DBN - 1) / DBN : 0);
     if ((int)blockIdx.y >= nbw) {  // pack rows [64 x, +64) of K quarter y - nbw (apack's code)
         const int nq = dense_pack_quarters(j.K), kq = (int)blockIdx.y - nbw;
         const int bpr = j.K / nq / 8, r0 = (int)blockIdx.x * DBM;  // blocks per row and quarter
@@ -97,16 +119,49 @@ __global__ __launch_bounds__(256 * KG) void dense_gemm_kernel(DenseJob j) {
     // row (never stored)
     const int sr = tid >> 2, sk = (tid & 3) * 16;
     const bf16_t *ap = j.A + (size_t)(row0 + min(sr, mrows - 1)) * j.lda + sk + kg * nks * DBK;
-    const bf16_t *bp = W + (size_t)min(n0 + sr, N - 1) * K + sk + kg * nks * DBK;
+    const size_t brow = (size_t)min(n0 + sr, N - 1);
+    const bf16_t *bp = W + brow * K + sk + kg * nks * DBK;
+    const QW &wq = second ? j.q1 : j.q0;
+    const uint8_t *cp = (const uint8_t *)wq.codes + brow * K + sk + kg * nks * DBK;
+    const int spk = Q8 ? wq.group / DBK : 1;  // K steps per scale
+    const bf16_t *sp = wq.scales + brow * (K / (Q8 ? wq.group : 1));
+    const bf16_t *zp = wq.biases ? wq.biases + brow * (K / (Q8 ? wq.group : 1)) : nullptr;
     // stages pass by value (a reference into them would put the ring in scratch)
     auto load = [&](int ks) __attribute__((always_inline)) -> Stage {
-        const uint4 *pa = (const uint4 *)(ap + ks * DBK), *pb = (const uint4 *)(bp + ks * DBK);
-        return Stage{pa[0], pa[1], pb[0], pb[1]};
+        const uint4 *pa = (const uint4 *)(ap + ks * DBK);
+        if constexpr (Q8) {
+            const int g = (kg * nks + ks) / spk;
+            const uint32_t sb = (uint32_t)sp[g] | (zp ? (uint32_t)zp[g] << 16 : 0u);
+            return Stage{pa[0], pa[1], *(const uint4 *)(cp + ks * DBK), uint4{}, sb};
+        } else {
+            const uint4 *pb = (const uint4 *)(bp + ks * DBK);
+            return Stage{pa[0], pa[1], pb[0], pb[1], 0u};
+        }
     };
     auto store = [&](int ks, Stage st) __attribute__((always_inline)) {
         bf16_t *a = &As[ks & 1][sr * DLDK + sk], *b = &Bs[ks & 1][sr * DLDK + sk];
         *(uint4 *)a = st.a0, *(uint4 *)(a + 8) = st.a1;
-        *(uint4 *)b = st.b0, *(uint4 *)(b + 8) = st.b1;
+        if constexpr (Q8) {
+            const uint2 p0 = q8_pairs(st.b0.x), p1 = q8_pairs(st.b0.y);
+            const uint2 p2 = q8_pairs(st.b0.z), p3 = q8_pairs(st.b0.w);
+            *(uint4 *)b = make_uint4(p0.x, p0.y, p1.x, p1.y);
+            *(uint4 *)(b + 8) = make_uint4(p2.x, p2.y, p3.x, p3.y);
+            float f[8], x = 0.f;
+            unpack8(st.a0, f);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x += f[i];
+            unpack8(st.a1, f);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x += f[i];
+            x = group_sum<4>(x);  // the row's four threads are one quad
+            if ((tid & 3) == 0) {
+                q8_lds[kg][ks & 1][0][sr] = x;
+                q8_lds[kg][ks & 1][1][sr] = bf_lo(st.sb);
+                q8_lds[kg][ks & 1][2][sr] = bf_hi(st.sb);
+            }
+        } else {
+            *(uint4 *)b = st.b0, *(uint4 *)(b + 8) = st.b1;
+        }
     };
 
     const int wm = wave >> 1, wn = wave & 1, fr = lane & 31, fk = (lane >> 5) * 8;
@@ -116,11 +171,26 @@ __global__ __launch_bounds__(256 * KG) void dense_gemm_kernel(DenseJob j) {
     auto compute = [&](int ks) __attribute__((always_inline)) {
         const bf16_t *a = &As[ks & 1][(wm * 32 + fr) * DLDK + fk];
         const bf16_t *b = &Bs[ks & 1][(wn * 32 + fr) * DLDK + fk];
+        f32x16_t part = {};
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+        for (int s = 0; s < 4; ++s) {
+            f32x16_t &c = Q8 ? part : acc;
+            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                 __builtin_bit_cast(bf16x8_t, *(const uint4 *)(a + 16 * s)),
-                __builtin_bit_cast(bf16x8_t, *(const uint4 *)(b + 16 * s)), acc, 0, 0, 0);
+                __builtin_bit_cast(bf16x8_t, *(const uint4 *)(b + 16 * s)), c, 0, 0, 0);
+        }
+        if constexpr (Q8) {
+            const float *q = &q8_lds[kg][ks & 1][0][0];
+            const float sc = q[DBM + wn * 32 + fr], bi = q[2 * DBM + wn * 32 + fr];
+#pragma unroll
+            for (int b4 = 0; b4 < 4; ++b4) {
+                const float4 x = *(const float4 *)(q + wm * 32 + 8 * b4 + 4 * (lane >> 5));
+                acc[4 * b4] += sc * part[4 * b4] + bi * x.x;
+                acc[4 * b4 + 1] += sc * part[4 * b4 + 1] + bi * x.y;
+                acc[4 * b4 + 2] += sc * part[4 * b4 + 2] + bi * x.z;
+                acc[4 * b4 + 3] += sc * part[4 * b4 + 3] + bi * x.w;
+            }
+        }
     };
     // ring slot i holds the loads of the steps = i (mod NST). Step ks (its tile in LDS buffer
     // ks & 1) issues its MFMAs, then stores step ks + 1's loads into the other buffer and refills
@@ -182,6 +252,11 @@ __global__ __launch_bounds__(256 * KG) void dense_gemm_kernel(DenseJob j) {
 
 bool dense_gemm_supported(int M, int K) { return M > 16 && K % DBK == 0 && K >= DBK; }
 
+bool dense_q8_supported(const QW &w) {
+    return w.codes && w.scales && w.bits == 8 && (w.group == 64 || w.group == 128) &&
+           ((uintptr_t)w.codes & 15) == 0 && w.in % DBK == 0;
+}
+
 // K groups of the launch: 2 measured best in the configs[2] prefill (router stage 18.0 against
 // 19.3 us with 1 group, 19.2 and 20.6 with 4 groups of 2- and 3-step rings) and with x in the
 // last-level cache (10.9 against 11.8 us, 4 groups 10.8); the steps wait on load latency, which
@@ -189,15 +264,22 @@ bool dense_gemm_supported(int M, int K) { return M > 16 && K % DBK == 0 && K >= 
 constexpr int kDenseKG = 2;
 
 hipError_t launch_dense_gemm(const DenseJob &j, hipStream_t stream) {
-    if (!dense_gemm_supported(j.M, j.K) || j.N0 <= 0 || (j.W1 && j.N1 <= 0))
+    const bool q8 = !j.W0;
+    if (!dense_gemm_supported(j.M, j.K) || j.N0 <= 0 || j.N1 < 0) return hipErrorInvalidValue;
+    if (q8 ? !dense_q8_supported(j.q0) || (j.N1 && (j.W1 || !dense_q8_supported(j.q1)))
+           : j.N1 && !j.W1)
         return hipErrorInvalidValue;
-    int nb = (j.N0 + DBN - 1) / DBN + (j.W1 ? (j.N1 + DBN - 1) / DBN : 0);
+    int nb = (j.N0 + DBN - 1) / DBN + (j.N1 + DBN - 1) / DBN;
     if (j.pack_a) nb += dense_pack_quarters(j.K);
     dim3 grid((j.M + DBM - 1) / DBM, nb);
     // a deeper ring (4, 6, 8 steps) measured no faster
-    if (j.K % (DBK * kDenseKG) == 0)
-        dense_gemm_kernel<3, kDenseKG><<<grid, 256 * kDenseKG, 0, stream>>>(j);
-    else dense_gemm_kernel<3, 1><<<grid, 256, 0, stream>>>(j);
+    if (j.K % (DBK * kDenseKG) == 0) {
+        if (q8) dense_gemm_kernel<3, kDenseKG, true><<<grid, 256 * kDenseKG, 0, stream>>>(j);
+        else dense_gemm_kernel<3, kDenseKG, false><<<grid, 256 * kDenseKG, 0, stream>>>(j);
+    } else {
+        if (q8) dense_gemm_kernel<3, 1, true><<<grid, 256, 0, stream>>>(j);
+        else dense_gemm_kernel<3, 1, false><<<grid, 256, 0, stream>>>(j);
+    }
     return hipGetLastError();
 }
 

@@ -250,8 +250,8 @@ struct DenseJob {
     int N0;
     bf16_t *out0;
     int ldo0;
-    const bf16_t *W1, *bias1;  // W1 null: none
-    int N1;
+    const bf16_t *W1, *bias1;
+    int N1;  // 0: none
     bf16_t *out1;
     int ldo1;
     uint32_t *zero;
@@ -260,8 +260,11 @@ struct DenseJob {
     // pack_x [M][3][K / pack_g]) by extra workgroups of the same launch
     bf16_t *pack_a, *pack_x;
     int pack_g;
+    QW q0, q1;  // W0 (and W1) null: 8-bit weights instead (dense_q8_supported)
 };
 bool dense_gemm_supported(int M, int K);
+// 8-bit weights launch_dense_gemm takes: groups of 64 or 128, in % 64 == 0
+bool dense_q8_supported(const QW &w);
 hipError_t launch_dense_gemm(const DenseJob &job, hipStream_t stream);
 
 // ---- elementwise ----

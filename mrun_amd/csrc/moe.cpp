@@ -302,6 +302,13 @@ static Status quantized_matmul(const bf16_t *x, int rows, const mrun_quantized &
     return Ok();
 }
 
+// A quantized Linear that the dense kernel runs: 8-bit, groups of 64 or 128, at most 512 outputs
+// (routers and gates: a launch of a few column blocks waits on latency, which that kernel's K
+// split and register ring shorten; wider products fill the GPU and stay on the generic GEMM).
+static bool linear_q8(const mrun_linear &l) {
+    return !l.weight && l.out <= 512 && dense_q8_supported(qw_of(l.q));
+}
+
 // Linear::forward (load.rs:294-306), dense or quantized. `zero` [n_zero] is cleared before the
 // product's results are visible to later launches (the prefill routing counters).
 static Status linear(const bf16_t *x, int rows, const mrun_linear &l, bf16_t *y, hipStream_t s,
@@ -311,6 +318,14 @@ static Status linear(const bf16_t *x, int rows, const mrun_linear &l, bf16_t *y,
         const bool mfma = dense_gemm_supported(rows, l.in) || (rows > 16 && !(l.out < 16) && l.in % 64 == 0);
         if (zero && !mfma) TRY_HIP(launch_fill_u32(zero, 0u, n_zero, s), "clear");
         return linear_dense(x, rows, l, y, s, mfma ? zero : nullptr, n_zero);
+    }
+    if (linear_q8(l) && dense_gemm_supported(rows, l.in)) {
+        DenseJob j{};
+        j.A = x, j.lda = l.in, j.M = rows, j.K = l.in;
+        j.q0 = qw_of(l.q), j.bias0 = l.bias, j.N0 = l.out, j.out0 = y, j.ldo0 = l.out;
+        j.zero = zero, j.n_zero = n_zero;
+        TRY_HIP(launch_dense_gemm(j, s), "linear (8-bit mfma)");
+        return Ok();
     }
     if (zero) TRY_HIP(launch_fill_u32(zero, 0u, n_zero, s), "clear");
     TRY(quantized_matmul(x, rows, l.q, y, s));
@@ -528,14 +543,18 @@ static Status sparse_moe_forward(const mrun_sparse_moe &m, const bf16_t *x, int 
     auto x_group = [](const mrun_quantized &q) { return q.bits != 16 && q.group_size == 32 ? 32 : 64; };
     const int xg = x_group(m.switch_gate_proj), og = x_group(m.switch_down_proj);
     const bool x_fits = p.x32 || (xg == 64 && og == 64);
-    if (m.gate.weight && (!S || m.shared_expert_gate.weight) && dense_gemm_supported(T, D)) {
+    const bool dense_gates = m.gate.weight && (!S || m.shared_expert_gate.weight);
+    const bool q8_gates = tensor::linear_q8(m.gate) && (!S || tensor::linear_q8(m.shared_expert_gate));
+    if ((dense_gates || q8_gates) && dense_gemm_supported(T, D)) {
         // router and shared gate: one launch over x
         DenseJob dj{};
         dj.A = x, dj.lda = D, dj.M = T, dj.K = D;
         dj.W0 = m.gate.weight, dj.bias0 = m.gate.bias, dj.N0 = E, dj.out0 = logits, dj.ldo0 = E;
+        if (q8_gates) dj.q0 = qw_of(m.gate.q);
         if (S) {
             dj.W1 = m.shared_expert_gate.weight, dj.bias1 = m.shared_expert_gate.bias;
             dj.N1 = 1, dj.out1 = sh_logit, dj.ldo1 = 1;
+            if (q8_gates) dj.q1 = qw_of(m.shared_expert_gate.q);
         }
         dj.zero = counts, dj.n_zero = p.n_counts;
         if (packs && x_fits) {
