@@ -308,6 +308,29 @@ struct F32Rows {
     float *out;
 };
 hipError_t launch_f32_rows(const F32Rows &j, bool glu, hipStream_t stream);
+// The same products for K <= 2048 with a wave's weight rows kept for every row that meets them.
+//  - Experts: expert active[i]'s rows are the pairs order[offsets[e] .. offsets[e + 1]); without
+//    routing (offsets null) slot i is pair i of expert ids[i]. Pair p reads A row p / a_div and
+//    writes out row p; W0, W1 [experts][N][K].
+//  - Plain rows (plain_rows > 0): pout[r] = pA[r] . pW0 (pW1) for r < plain_rows, in pieces of
+//    `piece` rows per workgroup; xW (no glu) is one more column, xout[r] = pA[r] . xW.
+// max_slots: experts (or pairs) in the launch. Every element has launch_f32_rows's bits.
+struct F32Group {
+    int K, N;
+    const float *A;
+    int a_div;
+    const float *W0, *W1;
+    float *out;
+    const uint32_t *ids, *offsets, *order, *active, *n_active;
+    const float *pA, *pW0, *pW1;
+    float *pout;
+    int plain_rows, piece;
+    const float *xW;
+    float *xout;
+    int plain_slots;  // set by the launcher
+};
+bool f32_group_supported(int K);
+hipError_t launch_f32_group(const F32Group &j, int max_slots, bool glu, hipStream_t stream);
 // softmax (f32) and top-k of T tokens (E <= 512; equal gates: lower id first; rank order); scores
 // are the gates, divided by their sum (in rank order) with norm
 hipError_t launch_f32_topk(const float *logits, int T, int E, int k, bool norm, uint32_t *ids,

@@ -843,6 +843,52 @@ static Status sparse_moe_forward_f32(const mrun_sparse_moe &m, const float *x, i
     uint32_t *ids = (uint32_t *)(ws + p.ids);
     float *act = (float *)(ws + p.act), *y = (float *)(ws + p.y);
     auto W = [](const mrun_quantized &q) { return (const float *)q.weight; };
+    float *sh_logit = S ? (float *)(ws + p.sh_logit) : nullptr, *sh_act = S ? (float *)(ws + p.sh_act) : nullptr;
+    float *sh_y = S ? (float *)(ws + p.sh_y) : nullptr;
+    // Grouped by expert once the batch holds a third of a pair per expert: the routing then takes
+    // the logits' place (dead after the top-k) where it fits there. With fewer pairs each is its own
+    // slot: few share an expert, and the sort's two launches take 11 us (Qwen3.6-like block, as
+    // pairs against grouped: T = 8, 64 pairs for 256 experts, 143.7 and 146.1 us; T = 12 209 and 202;
+    // T = 16 244 with half a pair per expert).
+    struct {
+        size_t counts, offsets, order, active, n_active, words;
+    } g{};
+    g.offsets = permute_counts_words(P, E), g.order = g.offsets + E + 1, g.active = g.order + P;
+    g.n_active = g.active + E, g.words = g.n_active + 1;
+    const bool kernels = f32_group_supported(D) && f32_group_supported(I) && (!S || S == I);
+    const bool group = kernels && 3 * P >= E && g.words <= (size_t)T * E;
+    if (kernels && (group || P <= 4096)) {
+        constexpr int kPiece = 8;  // plain rows per workgroup
+        F32Group r{};
+        r.K = D, r.N = E, r.pA = x, r.pW0 = W(m.gate.q), r.pout = logits, r.plain_rows = T, r.piece = kPiece;
+        if (S) r.xW = W(m.shared_expert_gate.q), r.xout = sh_logit;
+        TRY_HIP(launch_f32_group(r, 0, false, s), "f32 router");
+        TRY_HIP(launch_f32_topk(logits, T, E, k, c.norm_topk_prob != 0, ids, scores, s), "f32 top-k");
+        uint32_t *rt = (uint32_t *)logits;
+        F32Group gu{};
+        gu.ids = ids;
+        if (group) {
+            PermuteOut po{};
+            po.offsets = rt + g.offsets, po.order = rt + g.order, po.active = rt + g.active;
+            po.n_active = rt + g.n_active, po.tile_m = kGemmTileM;
+            TRY_HIP(launch_permute(ids, P, k, E, rt + g.counts, po, s), "f32 permute");
+            gu.offsets = po.offsets, gu.order = po.order, gu.active = po.active, gu.n_active = po.n_active;
+        }
+        const int slots = group ? (E < P ? E : P) : P;
+        F32Group dn = gu;
+        gu.K = D, gu.N = I, gu.A = x, gu.a_div = k, gu.out = act;
+        gu.W0 = W(m.switch_gate_proj), gu.W1 = W(m.switch_up_proj);
+        dn.K = I, dn.N = D, dn.A = act, dn.a_div = 1, dn.out = y, dn.W0 = W(m.switch_down_proj);
+        if (S) {
+            gu.pA = x, gu.pW0 = W(m.shared_gate_proj.q), gu.pW1 = W(m.shared_up_proj.q), gu.pout = sh_act;
+            dn.pA = sh_act, dn.pW0 = W(m.shared_down_proj.q), dn.pout = sh_y;
+            gu.plain_rows = dn.plain_rows = T, gu.piece = dn.piece = kPiece;
+        }
+        TRY_HIP(launch_f32_group(gu, slots, true, s), "f32 gate/up");
+        TRY_HIP(launch_f32_group(dn, slots, false, s), "f32 down");
+        TRY_HIP(launch_f32_combine(y, scores, T, k, D, sh_logit, sh_y, out, s), "f32 combine");
+        return Ok();
+    }
     // router: gates = softmax(gate(x)), top-k, scores (moe.rs:151-159)
     TRY_HIP(launch_f32_rows(F32Rows{x, 1, D, W(m.gate.q), nullptr, nullptr, T, E, logits}, false, s),
             "f32 router");
@@ -858,8 +904,6 @@ static Status sparse_moe_forward_f32(const mrun_sparse_moe &m, const float *x, i
     // the shared expert under its sigmoid gate (moe.rs:166-171)
     const float *gl = nullptr, *sy = nullptr;
     if (S > 0) {
-        float *sh_logit = (float *)(ws + p.sh_logit), *sh_act = (float *)(ws + p.sh_act),
-              *sh_y = (float *)(ws + p.sh_y);
         TRY_HIP(launch_f32_rows(F32Rows{x, 1, D, W(m.shared_expert_gate.q), nullptr, nullptr, T, 1,
                                         sh_logit},
                                 false, s),
