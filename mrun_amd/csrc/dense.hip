@@ -19,9 +19,9 @@
 // enters the result as  s * P + b * X  with X the step's sum of x, so no weight is rounded. The
 // launch reads half the dense router's bytes, and waits on the same latency: at 1000 tokens of the
 // Qwen3.6-like block the router, gate and packing took 48 us as four launches of the register-staged
-// GEMM of qgemm.hip (26 + 12), a fill (5) and the packing (5); one launch of this kernel took 32 us
-// off that block (313 -> 281 us per forward, 303 -> 269 at 2048 tokens of 4-bit experts, 158 -> 123
-// at 50).
+// GEMM of qgemm.hip (26 + 12), a fill (5) and the packing (5); one launch of this kernel takes 18.5
+// (22 with the scales' arithmetic at their loads): per forward of 4-bit experts 301 -> 273 us at 2048
+// tokens, 156 -> 115 at 50.
 //
 // With pack_a set, extra workgroups of the launch (column blocks past the product's, one per row
 // block and quarter of K) write A in the grouped GEMM's packed layout with launch_apack's code, bit
@@ -47,7 +47,8 @@ constexpr int DBM = 64, DBN = 64, DBK = 64, DLDK = DBK + 8;
 
 struct Stage {
     uint4 a0, a1, b0, b1;
-    uint32_t sb;  // Q8: the row's scale (low half) and bias of this K step, b0 its 16 codes
+    uint32_t sc, bi;  // Q8: the row's scale and bias of this K step (b0: its 16 codes), raw bits: any
+                      // arithmetic on them here would wait for the loads
 };
 
 // four 8-bit codes -> bf16 pairs (q0, q1), (q2, q3): integers below 256 are exact in bf16, so the
@@ -121,21 +122,24 @@ __global__ __launch_bounds__(256 * KG) void dense_gemm_kernel(DenseJob j) {
     const bf16_t *ap = j.A + (size_t)(row0 + min(sr, mrows - 1)) * j.lda + sk + kg * nks * DBK;
     const size_t brow = (size_t)min(n0 + sr, N - 1);
     const bf16_t *bp = W + brow * K + sk + kg * nks * DBK;
-    const QW &wq = second ? j.q1 : j.q0;
-    const uint8_t *cp = (const uint8_t *)wq.codes + brow * K + sk + kg * nks * DBK;
-    const int spk = Q8 ? wq.group / DBK : 1;  // K steps per scale
-    const bf16_t *sp = wq.scales + brow * (K / (Q8 ? wq.group : 1));
-    const bf16_t *zp = wq.biases ? wq.biases + brow * (K / (Q8 ? wq.group : 1)) : nullptr;
+    // Q8 (field by field: a reference to one of two kernel arguments would be read through memory)
+    const uint32_t *codes = second ? j.q1.codes : j.q0.codes;
+    const bf16_t *scales = second ? j.q1.scales : j.q0.scales;
+    const bf16_t *biases = second ? j.q1.biases : j.q0.biases;
+    const bf16_t *bptr = biases ? biases : scales;  // without biases: loaded, not used
+    const int gsh = (second ? j.q1.group : j.q0.group) == 128 ? 1 : 0;  // K steps per group, log2
+    const uint8_t *cp = (const uint8_t *)codes + brow * K + sk + kg * nks * DBK;
+    const size_t grow = brow * (size_t)((K / DBK) >> gsh);
     // stages pass by value (a reference into them would put the ring in scratch)
     auto load = [&](int ks) __attribute__((always_inline)) -> Stage {
         const uint4 *pa = (const uint4 *)(ap + ks * DBK);
         if constexpr (Q8) {
-            const int g = (kg * nks + ks) / spk;
-            const uint32_t sb = (uint32_t)sp[g] | (zp ? (uint32_t)zp[g] << 16 : 0u);
-            return Stage{pa[0], pa[1], *(const uint4 *)(cp + ks * DBK), uint4{}, sb};
+            const size_t g = grow + (size_t)((kg * nks + ks) >> gsh);
+            const uint32_t sc = scales[g], bi = bptr[g];
+            return Stage{pa[0], pa[1], *(const uint4 *)(cp + ks * DBK), uint4{}, sc, bi};
         } else {
             const uint4 *pb = (const uint4 *)(bp + ks * DBK);
-            return Stage{pa[0], pa[1], pb[0], pb[1], 0u};
+            return Stage{pa[0], pa[1], pb[0], pb[1], 0u, 0u};
         }
     };
     auto store = [&](int ks, Stage st) __attribute__((always_inline)) {
@@ -156,8 +160,8 @@ __global__ __launch_bounds__(256 * KG) void dense_gemm_kernel(DenseJob j) {
             x = group_sum<4>(x);  // the row's four threads are one quad
             if ((tid & 3) == 0) {
                 q8_lds[kg][ks & 1][0][sr] = x;
-                q8_lds[kg][ks & 1][1][sr] = bf_lo(st.sb);
-                q8_lds[kg][ks & 1][2][sr] = bf_hi(st.sb);
+                q8_lds[kg][ks & 1][1][sr] = bf2f(st.sc);
+                q8_lds[kg][ks & 1][2][sr] = biases ? bf2f(st.bi) : 0.f;
             }
         } else {
             *(uint4 *)b = st.b0, *(uint4 *)(b + 8) = st.b1;
