@@ -285,7 +285,7 @@ hipError_t launch_f32_group(const F32Group &j0, int max_slots, bool glu, hipStre
     j.plain_slots = j.plain_rows > 0 ? (j.plain_rows + j.piece - 1) / j.piece : 0;
     const int slots = j.plain_slots + max_slots;
     if (slots == 0 || j.N <= 0) return hipSuccess;
-    if (!f32_group_supported(j.K) || slots > 65535 || (glu && j.xW)) return hipErrorInvalidValue;
+    if (!f32_group_supported(j.K) || slots > kF32GroupMaxSlots || (glu && j.xW)) return hipErrorInvalidValue;
     if (glu) run_group<true>(j, slots, stream);
     else run_group<false>(j, slots, stream);
     return hipGetLastError();

@@ -330,6 +330,7 @@ struct F32Group {
     int plain_slots;  // set by the launcher
 };
 bool f32_group_supported(int K);
+constexpr int kF32GroupMaxSlots = 65535;  // pieces of plain rows and experts (or pairs): grid.y
 hipError_t launch_f32_group(const F32Group &j, int max_slots, bool glu, hipStream_t stream);
 // softmax (f32) and top-k of T tokens (E <= 512; equal gates: lower id first; rank order); scores
 // are the gates, divided by their sum (in rank order) with norm

@@ -857,8 +857,10 @@ static Status sparse_moe_forward_f32(const mrun_sparse_moe &m, const float *x, i
     g.n_active = g.active + E, g.words = g.n_active + 1;
     const bool kernels = f32_group_supported(D) && f32_group_supported(I) && (!S || S == I);
     const bool group = kernels && 3 * P >= E && g.words <= (size_t)T * E;
-    if (kernels && (group || P <= 4096)) {
-        constexpr int kPiece = 8;  // plain rows per workgroup
+    constexpr int kPiece = 8;  // plain rows per workgroup
+    const int slots = group ? (E < P ? E : P) : P;
+    const bool fits = (T + kPiece - 1) / kPiece + slots <= kF32GroupMaxSlots;
+    if (kernels && fits && (group || P <= 4096)) {
         F32Group r{};
         r.K = D, r.N = E, r.pA = x, r.pW0 = W(m.gate.q), r.pout = logits, r.plain_rows = T, r.piece = kPiece;
         if (S) r.xW = W(m.shared_expert_gate.q), r.xout = sh_logit;
@@ -874,7 +876,6 @@ static Status sparse_moe_forward_f32(const mrun_sparse_moe &m, const float *x, i
             TRY_HIP(launch_permute(ids, P, k, E, rt + g.counts, po, s), "f32 permute");
             gu.offsets = po.offsets, gu.order = po.order, gu.active = po.active, gu.n_active = po.n_active;
         }
-        const int slots = group ? (E < P ? E : P) : P;
         F32Group dn = gu;
         gu.K = D, gu.N = I, gu.A = x, gu.a_div = k, gu.out = act;
         gu.W0 = W(m.switch_gate_proj), gu.W1 = W(m.switch_up_proj);

@@ -5,6 +5,7 @@ from __future__ import annotations
 
 import numpy as np
 import pytest
+import torch
 
 from mrun_amd import moe as M
 from mrun_amd import synth
@@ -37,3 +38,13 @@ def test_rows_do_not_depend_on_the_grouping(shape):
         part = dev.forward(f32_dev(x[:T])).cpu().numpy().view(np.uint32)
         assert np.array_equal(part, full[:T]), T
     check(fb, dev, x, shape.name)
+
+
+def test_more_row_pieces_than_a_grid_holds():
+    """530,000 rows are 66,250 pieces: the per-row kernel runs them, with the same bits."""
+    shape = synth.Shape(hidden=32, experts=4, top_k=1, intermediate=32, shared=32)
+    dev = M.SparseMoeF32(synth.make_block_f32(shape, config=29))
+    x = f32_dev(synth.make_x_f32(shape, 1000, config=29)).repeat(530, 1)
+    full = dev.forward(x)
+    part = dev.forward(x[:1000].contiguous())
+    assert torch.equal(full.view(530, 1000, 32), part.expand(530, -1, -1))
