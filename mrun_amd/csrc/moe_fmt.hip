@@ -10,8 +10,11 @@
 // memory straight into an LDS ring, the next stage in flight while one is computed; the affine
 // dequant folded around v_mfma_f32_32x32x16_bf16, no weight rounded), with these differences:
 //  - A stage holds 64 or 128 bytes of each weight row: two K steps (of 64) of 4-bit codes, one of
-//    8-bit codes, or one of bf16 weights (whole 128-byte lines). 32-row tiles of 8-bit experts run
-//    a ring of three stages.
+//    8-bit codes, or one of bf16 weights (whole 128-byte lines). Where a stage is at
+//    most 24 KB (8-bit codes, and 4-bit ones in 32-row tiles) the ring has three: the scales then
+//    go to registers, a chunk ahead, which frees their LDS (8-bit T = 1000 269.8 -> 262.0 us, group
+//    32 T = 700 241.6 -> 233.2). With two stages they stay in LDS (in registers, group 128 T = 1200
+//    took 197 us for 191).
 //  - 8-bit codes become exact bf16 integers (no offset); each dword holds codes i and i + 4 of a
 //    block, as the packed A has them. bf16 weights are re-paired the same way and go to the MFMAs
 //    without scales, straight into the accumulators.
@@ -41,17 +44,19 @@ template <int NMI, int BITS, int GROUP>
 struct FmtCfg {
     static constexpr bool QUANT = BITS != 16;
     static constexpr int KS = BITS == 4 ? 2 : 1;         // K steps of 64 per stage
-    static constexpr int NSTG = BITS == 8 && NMI == 1 ? 3 : 2;
     static constexpr int A_STEP = NMI * 32 * 128, A_BYTES = KS * A_STEP;
     static constexpr int C_ROW = BITS * 8 * KS;          // bytes of a weight row per stage
     static constexpr int C_BYTES = 256 * C_ROW;
     static constexpr int STAGE = A_BYTES + C_BYTES;
+    static constexpr int NSTG = STAGE <= 24576 ? 3 : 2;  // what two workgroups per CU leave room for
     static constexpr int A_PARTS = KS * NMI, C_PARTS = C_BYTES / 4096, PARTS = A_PARTS + C_PARTS;
     static constexpr int C_RPP = 256 / C_PARTS;          // weight rows per copy part
     static constexpr int CH = GROUP == 32 ? 4 : 8;       // K steps per chunk of scales and biases
     static constexpr int XG = GROUP == 32 ? 32 : 64;     // inputs per X sum
-    static constexpr int S_BYTES = QUANT ? 4096 : 0;     // 8 (group 128: 4) scales per weight row
-    static constexpr int X_BYTES = QUANT ? 3 * 64 * 16 : 0, B_BYTES = S_BYTES;
+    // with three stages a chunk's scales wait in registers, else in LDS: 8 (group 128: 4) per row
+    static constexpr bool SREG = NSTG == 3;
+    static constexpr int B_BYTES = QUANT ? 4096 : 0, S_BYTES = SREG ? 0 : B_BYTES;
+    static constexpr int X_BYTES = QUANT ? 3 * 64 * 16 : 0;
     static constexpr int OFF_S = NSTG * STAGE, OFF_R = OFF_S + 2 * S_BYTES;
     static constexpr int OFF_T = OFF_R + 512, OFF_X = OFF_T + 512, OFF_B = OFF_X + X_BYTES;
     static constexpr int LDS_BYTES = OFF_B + B_BYTES;
@@ -182,9 +187,10 @@ __global__ __launch_bounds__(256, 2) void fmt_gemm_kernel(MoeGemmJob j) {
     constexpr int UPR = C::C_ROW / 16;  // 16-byte units of a weight row per stage: 4 or 8
     const int rb = wave * (64 / UPR) + lane / UPR;
     const uint32_t uc16 = 16u * (uint32_t)((lane % UPR) ^ (UPR == 8 ? swz_a(rb) : swz_c(rb)));
-    rsrc_t r_a, r_c0, r_c1, r_s;
-    uint32_t la0 = 0, la1 = 0, lc = 0, ls = 0;
+    rsrc_t r_a, r_c0, r_c1, r_s0, r_s1;
+    uint32_t la0 = 0, la1 = 0, lc = 0, ls0 = 0, ls1 = 0;
     int l_item = 0, l_ks = 0, l_chunk = 0, l_slot = 0;
+    u32x4 sn0 = {0u, 0u, 0u, 0u}, sn1 = sn0;  // SREG: this lane's two rows' scales of the load cursor's chunk
     Item li{};   // the load cursor's item, taken over by the compute cursor at its switch
     int lx = 0;  // the load cursor's A row of tile row `lane` (the bias term's X splits)
 
@@ -208,11 +214,16 @@ __global__ __launch_bounds__(256, 2) void fmt_gemm_kernel(MoeGemmJob j) {
         r_c1 = GLU ? rsrc_of(it.sh ? j.sh.w1.codes : j.w1.codes) : r_c0;
         const uint32_t wrow = (uint32_t)it.e * (uint32_t)j.N + (uint32_t)it.n0;
         lc = (wrow + (uint32_t)rb) * row_bytes + uc16;
-        if (C::QUANT) {  // weight row tid: gate rows then up rows under glu
+        if (C::QUANT && !C::SREG) {  // weight row tid: gate rows then up rows under glu
             const bool up = GLU && wave >= 2;
-            r_s = rsrc_of(up ? (it.sh ? j.sh.w1.scales : j.w1.scales)
-                             : (it.sh ? j.sh.w0.scales : j.w0.scales));
-            ls = (wrow + (uint32_t)(GLU ? (tid & 127) : tid)) * (uint32_t)G * 2u;
+            r_s0 = rsrc_of(up ? (it.sh ? j.sh.w1.scales : j.w1.scales)
+                              : (it.sh ? j.sh.w0.scales : j.w0.scales));
+            ls0 = (wrow + (uint32_t)(GLU ? (tid & 127) : tid)) * (uint32_t)G * 2u;
+        } else if (C::QUANT) {  // weight rows bro0 + fr and bro1 + fr of the compute role
+            r_s0 = rsrc_of(it.sh ? j.sh.w0.scales : j.w0.scales);
+            r_s1 = GLU ? rsrc_of(it.sh ? j.sh.w1.scales : j.w1.scales) : r_s0;
+            ls0 = (wrow + (uint32_t)((GLU ? 32 : 64) * wave + fr)) * (uint32_t)G * 2u;
+            ls1 = GLU ? ls0 : ls0 + 64u * (uint32_t)G;
         }
         fetch_rows(n + 1);
     };
@@ -244,8 +255,18 @@ __global__ __launch_bounds__(256, 2) void fmt_gemm_kernel(MoeGemmJob j) {
     };
     auto begin_stage = [&]() __attribute__((always_inline)) {  // before a stage's copies
         if (C::QUANT && l_ks % C::CH == 0) {
-            copy_chunk(r_s, ls, l_ks / C::CH, smem + C::OFF_S + (l_chunk & 1) * C::S_BYTES);
-            ++l_chunk;
+            const uint32_t c = (uint32_t)(l_ks / C::CH);
+            if constexpr (!C::SREG) {
+                copy_chunk(r_s0, ls0, (int)c, smem + C::OFF_S + (l_chunk & 1) * C::S_BYTES);
+                ++l_chunk;
+            } else if constexpr (GROUP == 128) {
+                const u32x2 v0 = __builtin_amdgcn_raw_buffer_load_b64(r_s0, ls0, 8u * c, 0);
+                const u32x2 v1 = __builtin_amdgcn_raw_buffer_load_b64(r_s1, ls1, 8u * c, 0);
+                sn0.x = v0.x, sn0.y = v0.y, sn1.x = v1.x, sn1.y = v1.y;
+            } else {
+                sn0 = __builtin_amdgcn_raw_buffer_load_b128(r_s0, ls0, 16u * c, 0);
+                sn1 = __builtin_amdgcn_raw_buffer_load_b128(r_s1, ls1, 16u * c, 0);
+            }
         }
     };
     // the load cursor's next stage (and item; past the last it stays on that item, in bounds)
@@ -388,6 +409,10 @@ __global__ __launch_bounds__(256, 2) void fmt_gemm_kernel(MoeGemmJob j) {
                            smem + C::OFF_B);
             }
         }
+        if (C::QUANT && C::SREG && ST == 0 && ks % C::CH == 0) {  // the chunk's scales, before the next are loaded
+            if constexpr (GROUP == 128) sch0 = fmt_dup(sn0.x, sn0.y), sch1 = fmt_dup(sn1.x, sn1.y);
+            else sch0 = sn0, sch1 = sn1;
+        }
         // the load cursor moves on after the stage it last issued
         if constexpr (!SS || C::KS == 1) advance();
         if constexpr (SS) begin_stage();
@@ -437,7 +462,7 @@ __global__ __launch_bounds__(256, 2) void fmt_gemm_kernel(MoeGemmJob j) {
                      [q0] "v"(pc[0]), [q1] "v"(pc[NCA > 1 ? 1 : 0]), [q2] "v"(pc[NCA > 2 ? 2 : 0]),
                      [q3] "v"(pc[NCA > 3 ? 3 : 0]), [db] "i"(DB * C::C_ROW));
         }
-        if (C::QUANT && ST == 0 && ks % C::CH == 0) {  // the chunk's scales
+        if (C::QUANT && !C::SREG && ST == 0 && ks % C::CH == 0) {  // the chunk's scales
             ++c_chunk;
             const uint32_t sp = lds0 + C::OFF_S + (uint32_t)((c_chunk & 1) * C::S_BYTES);
             if constexpr (GROUP == 128) {
