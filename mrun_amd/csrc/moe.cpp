@@ -398,7 +398,11 @@ struct FusedNorm {
 // rows for the grouped GEMM. On the configs[1] block (per block, 32- against 64-row tiles):
 // T = 33 131 -> 111 us, 64 154 -> 132, 128 164 -> 144, 256 180 -> 159, 512 190 -> 165, 768 199 ->
 // 179; T = 1024 (32 rows on average) the same; T = 2048 281 -> 308 (Zipf router: 268 -> 311).
-constexpr int kHalfTileMaxRows = 28;
+// 4-bit experts in groups of 32 or 128 (moe_fmt.hip), whose 32-row tiles run the longer ring, go on
+// to 32 rows: group 32 T = 900 (28.1 rows) 275 -> 233 us, T = 1200 (37.5 rows) 270 -> 280 (with the
+// even split of both), group 128 T = 900 192 -> 171, 1050 193 -> 191, 1200 197 -> 213. 8-bit experts
+// as group 64: T = 900 257 against 258, T = 1000 259 -> 271.
+constexpr int kHalfTileMaxRows = 28, kHalfTileMaxRowsFmt4 = 32;
 
 // the largest batch that runs as decode-schedule chunks of at most 16 tokens, when the decode
 // kernels do not take it whole (more than 256 pairs: k above 8)
@@ -575,7 +579,9 @@ static Status sparse_moe_forward(const mrun_sparse_moe &m, const bf16_t *x, int 
     // mid-size batches: the routed tiles cut to 32 rows (most experts hold a few rows, so a 64-row
     // tile is mostly padding), on the grouped GEMM's one-row-fragment instantiation; bf16 experts
     // run 32-row tiles at every size
-    const bool half = (long long)P <= (long long)kHalfTileMaxRows * E ||
+    const mrun_quantized &gp = m.switch_gate_proj;
+    const int half_rows = gp.bits == 4 && gp.group_size != 64 ? kHalfTileMaxRowsFmt4 : kHalfTileMaxRows;
+    const bool half = (long long)P <= (long long)half_rows * E ||
                       m.switch_gate_proj.bits == 16 || m.switch_down_proj.bits == 16;
     // the grouped GEMM (moe_gemm.hip, moe_fmt.hip): K a multiple of 512, the shared expert in the
     // same launches when its width and format equal the routed ones
