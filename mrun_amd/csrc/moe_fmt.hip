@@ -127,9 +127,22 @@ __global__ __launch_bounds__(256, 2) void fmt_gemm_kernel(MoeGemmJob j) {
     const int r_tiles =
         j.has_routing ? min((int)*j.routing.n_tiles, j.max_tiles) : (j.M + TM - 1) / TM;
     const int total = (s_tiles + r_tiles) * NB;
-    const int G8 = (int)(gridDim.x >> 3), xcd = (int)(blockIdx.x & 7), wg = (int)(blockIdx.x >> 3);
+    const int G0 = (int)(gridDim.x >> 3), xcd = (int)(blockIdx.x & 7), wg = (int)(blockIdx.x >> 3);
     const int seg_lo = (int)((long long)total * xcd / 8);
     const int seg_hi = (int)((long long)total * (xcd + 1) / 8);
+    // Up to three items per workgroup: as many workgroups as share the XCD's items evenly (136 items
+    // on 64 workgroups: 46 with three each, not 8 with three and 56 with two), for the gate/up
+    // products of bf16 weights and of groups of 32. Each workgroup streams whole lines of 256 weight
+    // rows (and, for groups of 32, of their scales and biases, 16 bytes of a line at a time), so
+    // fewer of them keep those lines in the XCD's L2: bf16 T = 200 / 300 / 600 342 -> 322, 388 -> 351,
+    // 395 -> 364 us per block, group 32 T = 200 / 700 / 1600 207 -> 194, 221 -> 211, 302 -> 291. The
+    // other formats need the loads in flight (8-bit T = 700 236 -> 247 us, group 128 157 -> 163), the
+    // down products measured the same, and with more items the last round is a small part (group 32
+    // T = 3000 423 -> 435, bf16 T = 2000 490 -> 492).
+    constexpr bool EVEN = GLU && (!C::QUANT || GROUP == 32) && BITS != 8;
+    const int rounds = (seg_hi - seg_lo + G0 - 1) / G0;
+    const int G8 = uni(EVEN && rounds > 1 && rounds <= 3 ? (seg_hi - seg_lo + rounds - 1) / rounds : G0);
+    if (EVEN && wg >= G8) return;
     const int n_items = uni(seg_hi - seg_lo > wg ? (seg_hi - seg_lo - wg + G8 - 1) / G8 : 0);
     if (n_items == 0) return;
     const int K = j.K, nks = K / 64, G = K / GROUP, axe = K / C::XG;

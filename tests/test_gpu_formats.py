@@ -88,3 +88,16 @@ def test_gather_qmm(bits, group):
     got = M.bf16_bits(M.gather_qmm(M.bf16_tensor(x), M.DeviceQTensor(q), M.u32_tensor(ids)))
     ref = O.gather_qmm(q, x, ids)
     assert_close(got, ref, what=f"gather_qmm {bits}-bit group {group}")
+
+
+@pytest.mark.parametrize("T", [900, 1500, 2600, 6000])
+@pytest.mark.parametrize("bits,group", [(4, 32), (8, 64), (16, 64)])
+def test_rows_keep_their_bits_across_item_rounds(bits, group, T):
+    """Workgroups that take one to six items each, split evenly over fewer workgroups or not: every
+    row as in a batch of one item per workgroup."""
+    hb = _host(bits, group, layer=8, intermediate=1024, shared=1024)
+    dev = M.SparseMoe(hb)
+    x = np.resize(_x(hb.shape, 97), (T, hb.shape.hidden))
+    full = M.bf16_bits(dev.forward(M.bf16_tensor(x)))
+    part = M.bf16_bits(dev.forward(M.bf16_tensor(x[:97])))
+    assert np.array_equal(full, np.resize(part, full.shape))
