@@ -24,9 +24,9 @@
 //  - Groups of 128: the two K steps of a group apply the same scale; the X sums stay per 64.
 //  - The LDS reads of a K step and their wait are one asm statement.
 // Measured on the Qwen3.6-like block, whole forwards, against the register-staged GEMM of qgemm.hip
-// (64 x 64 tiles, the shared expert in two launches of its own): 8-bit experts T = 1000 471 -> 313
-// us, 4-bit group 32 T = 700 559 -> 285, group 128 T = 200 331 -> 185, bf16 T = 300 677 -> 353
-// (1.6 GB of weights: 4.6 TB/s, the rate of a large copy) and T = 2000 1005 -> 468.
+// (64 x 64 tiles, the shared expert in two launches of its own): 8-bit experts T = 1000 472 -> 265
+// us, 4-bit group 32 T = 700 545 -> 222, bf16 T = 300 676 -> 342 (1.6 GB of weights: 4.7 TB/s, near
+// the rate of a large copy).
 #include <type_traits>
 
 #include "apack.hpp"
