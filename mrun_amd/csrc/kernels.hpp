@@ -211,7 +211,7 @@ struct MoeGemmJob {
     QW w0, w1;
     Routing routing;
     int has_routing, max_tiles;
-    int tile_m;  // rows per tile: 64, or 32 (the routed tiles cut to 32 rows by the permute)
+    int tile_m;  // rows per tile: 64 (or 0), or 32 (the routed tiles cut to 32 rows by the permute)
     int M;
     bf16_t *out;
     int ldo;

@@ -1216,8 +1216,9 @@ int mrun_gather_qmm(const mrun_bf16 *x, int32_t x_rows, const mrun_quantized *w,
         po.n_active = u32(p.n_active), po.tiles = u32(p.tiles), po.n_tiles = u32(p.n_tiles);
         po.tile_m = kGemmTileM;
         Routing rt{po.offsets, po.active, po.n_active, po.tiles, po.n_tiles};
-        // the tuned grouped GEMM (4-bit group 64, in % 512, out % 256): x packed, the tiles' x
-        // rows from the permute, the product in expert order, then each index's row in place
+        // the tuned grouped GEMM (4- and 8-bit, groups of 64 and 128: the plan holds sums of 64 inputs
+        // and 64-row tiles; in % 512, out % 256): x packed, the tiles' x rows from the permute, the
+        // product in expert order, then each index's row in place
         MoeGemmJob mj{};
         if (n > 16) {
             mj.A = (const bf16_t *)(ws + p.xp), mj.lda = w->in, mj.a_rows = x_rows;

@@ -692,7 +692,7 @@ bool fmt_gemm_supported(const MoeGemmJob &j) {
     if (w0.bits != 4 && w0.bits != 8 && w0.bits != 16) return false;
     if (quant && w0.group != 32 && w0.group != 64 && w0.group != 128) return false;
     if (j.K % 512 != 0 || !pair_ok(w0, j.w1) || (j.has_shared && !pair_ok(j.sh.w0, j.sh.w1))) return false;
-    if (!quant && j.tile_m == 64) return false;  // bf16 weights: 32-row tiles
+    if (!quant && j.tile_m != 32) return false;  // bf16 weights: 32-row tiles only (0 is 64)
     const int xg = w0.group == 32 ? 32 : 64;     // X sums of the A rows
     if (quant && (j.ax_g != xg || j.ax_e != j.K / xg)) return false;
     if (j.glu) {  // X sums of act for the down product

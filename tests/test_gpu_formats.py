@@ -78,16 +78,18 @@ def test_mixed_formats(gate, down):
         run_block(hb, M.SparseMoe(hb), _x(hb.shape, T), f"gate/up {gate} down {down} T={T}")
 
 
-@pytest.mark.parametrize("bits,group", [(8, 64), (4, 128)])
-def test_gather_qmm(bits, group):
-    """gather_qmm above 16 indices on the grouped GEMM: unsorted indices, x rows shared by two."""
-    q = _host(bits, group, layer=6).gate_proj
+# 1024 inputs: the grouped GEMM (groups of 32 and bf16 weights: the generic one); 640: the generic one
+@pytest.mark.parametrize("hidden", [1024, 640])
+@pytest.mark.parametrize("bits,group", [(4, 64)] + FORMATS)
+def test_gather_qmm(bits, group, hidden):
+    """gather_qmm above 16 indices in every format: unsorted indices, x rows shared by two."""
+    q = _host(bits, group, layer=6, hidden=hidden).gate_proj
     n, rows = 150, 75
     ids = np.random.default_rng(1).integers(0, q.experts, n).astype(np.uint32)
     x = _x(synth.Shape(q.in_, 1, 1, 32), rows)
     got = M.bf16_bits(M.gather_qmm(M.bf16_tensor(x), M.DeviceQTensor(q), M.u32_tensor(ids)))
     ref = O.gather_qmm(q, x, ids)
-    assert_close(got, ref, what=f"gather_qmm {bits}-bit group {group}")
+    assert_close(got, ref, what=f"gather_qmm {bits}-bit group {group} in {hidden}")
 
 
 @pytest.mark.parametrize("T", [900, 1500, 2600, 6000])
