@@ -624,10 +624,15 @@ __global__ __launch_bounds__(256, 2) void fmt_gemm_kernel(MoeGemmJob j) {
         }
         if (ST != 3 || ks != nks - 1) return;
         if constexpr (C::QUANT) {  // the item's last scale
+            // the products are cleared with the scale: the next item's first step adds 0 times them,
+            // which an infinity or NaN of one of this item's rows would turn into NaN there
 #pragma unroll
             for (int mi = 0; mi < NMI; ++mi)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) acc[mi][1][i] += sc_pend * part[1][mi][i];
+                for (int i = 0; i < 16; ++i) {
+                    acc[mi][1][i] += sc_pend * part[1][mi][i];
+                    part[1][mi][i] = 0.f;
+                }
             sc_pend = 0.f;
         }
 

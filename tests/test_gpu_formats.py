@@ -103,3 +103,22 @@ def test_rows_keep_their_bits_across_item_rounds(bits, group, T):
     full = M.bf16_bits(dev.forward(M.bf16_tensor(x)))
     part = M.bf16_bits(dev.forward(M.bf16_tensor(x[:97])))
     assert np.array_equal(full, np.resize(part, full.shape))
+
+
+# 6,000 rows of 8 experts: three rounds of 64-row tiles per workgroup; 400 rows of 128 experts (25
+# rows each): more 32-row tiles than workgroups
+@pytest.mark.parametrize("T,kw", [(6000, {}), (400, dict(hidden=512, experts=128, top_k=8))])
+@pytest.mark.parametrize("bits,group", FORMATS)
+def test_a_non_finite_row_stays_alone(bits, group, T, kw):
+    """A token row of infinities or NaN (an uninitialised padding row) changes no other row: nothing
+    of one tile's products reaches the next tile of the same workgroup."""
+    hb = _host(bits, group, layer=9, **kw)
+    dev = M.SparseMoe(hb)
+    x = np.resize(_x(hb.shape, 97), (T, hb.shape.hidden))
+    clean = M.bf16_bits(dev.forward(M.bf16_tensor(x)))
+    bad = np.array([3, T // 2, T - 5])
+    x[bad] = np.array([0x7F80, 0xFF80, 0x7FC0], dtype=np.uint16)[:, None]  # inf, -inf, NaN
+    got = M.bf16_bits(dev.forward(M.bf16_tensor(x)))
+    others = np.setdiff1d(np.arange(T), bad)
+    wrong = others[np.any(got[others] != clean[others], axis=1)]
+    assert wrong.size == 0, f"{wrong.size} other rows changed, the first {wrong[:4]}"
