@@ -483,11 +483,16 @@ __global__ __launch_bounds__(mg::NT, 2) void moe_gemm_kernel(MoeGemmJob j) {
             }
         }
         if (ST != 3 || ks != nks - 1) return;
-        // the item's last fragment-1 scale
+        // the item's last fragment-1 scale. The products are cleared with the scale: the next item's
+        // first step adds 0 times them, which an infinity or NaN of one of this item's rows would
+        // turn into NaN there.
 #pragma unroll
         for (int mi = 0; mi < NMI; ++mi)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) acc[mi][1][i] += sc_pend * part1[mi][i];
+            for (int i = 0; i < 16; ++i) {
+                acc[mi][1][i] += sc_pend * part1[mi][i];
+                part1[mi][i] = 0.f;
+            }
         sc_pend = 0.f;
 
         // ---- epilogue of item ci. Stores are widened by exchanging values between lanes (DPP):
