@@ -4,11 +4,14 @@
 // f32: nothing is rounded to bf16, and the SwiGLU's casts (activations.rs:64-66) are identities.
 //
 // Every output element is one wave's dot product over float4 loads, with a fixed reduction order, so
-// a row's result does not depend on the batch. Inputs of up to 2048 run f32_group_kernel: a wave
-// keeps ND weight rows in registers (64 of them at most) and takes every row that meets them, so an
-// expert's weights are read once per batch, not once per pair (bound by streaming them: the
-// Qwen3.6-like block in f32 holds 12.6 MB per expert). Wider inputs run f32_rows_kernel, one dot
-// product per wave, whose bits are the same.
+// a row's result does not depend on the batch. Widths of up to 2048, with a shared expert as wide as
+// the routed ones or none, run f32_group_kernel: a wave keeps ND weight rows in registers (64 of them
+// at most) and takes the rows of a tile that meets them, one after the other, so an expert's weights
+// are read once per tile of 8 to 64 of its rows, not once per pair (bound by streaming them: the
+// Qwen3.6-like block in f32 holds 12.6 MB per expert). Tiles, because a wave takes about 0.6 us per
+// row: with all of an expert's rows in one wave, 16 experts of width 256 x 128 took 590 us at T = 2048
+// (537 as single dot products, 134 in tiles of 8). Other blocks run f32_rows_kernel, one dot product
+// per wave, whose bits are the same.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -99,7 +102,7 @@ __device__ __forceinline__ float wave_sums(const float (&v)[ND], int lane) {
 }
 
 // The products of F32Group (kernels.hpp). Slot blockIdx.y: first the plain rows in pieces of
-// j.piece, then the experts' (or single pairs'). A wave owns NW = ND (glu: ND / 2) output columns.
+// j.piece, then the experts' tiles (or single pairs). A wave owns NW = ND (glu: ND / 2) output columns.
 template <bool GLU, int NC, int ND>
 __global__ __launch_bounds__(256) void f32_group_kernel(F32Group j) {
     constexpr int NW = GLU ? ND / 2 : ND;
@@ -118,10 +121,10 @@ __global__ __launch_bounds__(256) void f32_group_kernel(F32Group j) {
     } else {
         s -= j.plain_slots;
         int e;
-        if (j.offsets) {
-            if (s >= (int)*j.n_active) return;
-            e = (int)j.active[s];
-            p0 = (int)j.offsets[e], rows = (int)j.offsets[e + 1] - p0, map = j.order;
+        if (j.tiles) {
+            if (s >= (int)*j.n_tiles) return;
+            e = (int)j.tiles[3 * s], p0 = (int)j.tiles[3 * s + 1], rows = (int)j.tiles[3 * s + 2];
+            map = j.order;
         } else {
             e = (int)j.ids[s], p0 = s, rows = 1;
         }
@@ -268,11 +271,16 @@ hipError_t launch_f32_rows(const F32Rows &j, bool glu, hipStream_t stream) {
 }
 
 // Weight rows per wave by input width, so that a wave holds at most 64 registers of weights.
+static int group_nd(int K) { return K > 1024 ? 2 : K > 512 ? 4 : 8; }
+
+int f32_group_blocks(int K, int N, bool glu) {
+    const int cols = 4 * (glu ? group_nd(K) / 2 : group_nd(K));
+    return (N + cols - 1) / cols;
+}
+
 template <bool GLU>
 static void run_group(const F32Group &j, int slots, hipStream_t s) {
-    const int nd = j.K > 1024 ? 2 : j.K > 512 ? 4 : 8, nw = GLU ? nd / 2 : nd;
-    const int cols = j.N + (j.xW ? 1 : 0);
-    const dim3 grid((cols + 4 * nw - 1) / (4 * nw), slots);
+    const dim3 grid(f32_group_blocks(j.K, j.N + (j.xW ? 1 : 0), GLU), slots);
     if (j.K > 1024) f32_group_kernel<GLU, 8, 2><<<grid, 256, 0, s>>>(j);
     else if (j.K > 512) f32_group_kernel<GLU, 4, 4><<<grid, 256, 0, s>>>(j);
     else f32_group_kernel<GLU, 2, 8><<<grid, 256, 0, s>>>(j);

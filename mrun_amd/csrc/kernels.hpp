@@ -309,19 +309,19 @@ struct F32Rows {
 };
 hipError_t launch_f32_rows(const F32Rows &j, bool glu, hipStream_t stream);
 // The same products for K <= 2048 with a wave's weight rows kept for every row that meets them.
-//  - Experts: expert active[i]'s rows are the pairs order[offsets[e] .. offsets[e + 1]); without
-//    routing (offsets null) slot i is pair i of expert ids[i]. Pair p reads A row p / a_div and
-//    writes out row p; W0, W1 [experts][N][K].
+//  - Experts: slot i < n_tiles is tile i = tiles[3 i ..] (expert, first row, rows): the pairs
+//    order[first ..] (PermuteOut's tiles); without routing (tiles null) slot i is pair i of expert
+//    ids[i]. Pair p reads A row p / a_div and writes out row p; W0, W1 [experts][N][K].
 //  - Plain rows (plain_rows > 0): pout[r] = pA[r] . pW0 (pW1) for r < plain_rows, in pieces of
 //    `piece` rows per workgroup; xW (no glu) is one more column, xout[r] = pA[r] . xW.
-// max_slots: experts (or pairs) in the launch. Every element has launch_f32_rows's bits.
+// max_slots: tiles (or pairs) in the launch. Every element has launch_f32_rows's bits.
 struct F32Group {
     int K, N;
     const float *A;
     int a_div;
     const float *W0, *W1;
     float *out;
-    const uint32_t *ids, *offsets, *order, *active, *n_active;
+    const uint32_t *ids, *order, *tiles, *n_tiles;
     const float *pA, *pW0, *pW1;
     float *pout;
     int plain_rows, piece;
@@ -330,7 +330,9 @@ struct F32Group {
     int plain_slots;  // set by the launcher
 };
 bool f32_group_supported(int K);
-constexpr int kF32GroupMaxSlots = 65535;  // pieces of plain rows and experts (or pairs): grid.y
+// workgroups that cover N columns of one slot, for inputs of width K
+int f32_group_blocks(int K, int N, bool glu);
+constexpr int kF32GroupMaxSlots = 65535;  // pieces of plain rows and tiles (or pairs): grid.y
 hipError_t launch_f32_group(const F32Group &j, int max_slots, bool glu, hipStream_t stream);
 // softmax (f32) and top-k of T tokens (E <= 512; equal gates: lower id first; rank order); scores
 // are the gates, divided by their sum (in rank order) with norm

@@ -851,22 +851,36 @@ static Status sparse_moe_forward_f32(const mrun_sparse_moe &m, const float *x, i
     auto W = [](const mrun_quantized &q) { return (const float *)q.weight; };
     float *sh_logit = S ? (float *)(ws + p.sh_logit) : nullptr, *sh_act = S ? (float *)(ws + p.sh_act) : nullptr;
     float *sh_y = S ? (float *)(ws + p.sh_y) : nullptr;
-    // Grouped by expert once the batch holds a third of a pair per expert: the routing then takes
-    // the logits' place (dead after the top-k) where it fits there. With fewer pairs each is its own
-    // slot: few share an expert, and the sort's two launches take 11 us (Qwen3.6-like block, as
-    // pairs against grouped: T = 8, 64 pairs for 256 experts, 143.7 and 146.1 us; T = 12 209 and 202;
-    // T = 16 244 with half a pair per expert).
-    struct {
-        size_t counts, offsets, order, active, n_active, words;
-    } g{};
-    g.offsets = permute_counts_words(P, E), g.order = g.offsets + E + 1, g.active = g.order + P;
-    g.n_active = g.active + E, g.words = g.n_active + 1;
+    // Sorted by expert (an expert's weights then meet its rows in tiles of up to tile_m), the routing
+    // in the logits' place (dead after the top-k) where it fits; else every pair is its own slot, and
+    // reads its expert's weights by itself. The sort's two launches take 8 to 11 us, about what 400 MB
+    // of weights cost the pairs from the caches (us as pairs and sorted; 3 D I floats per pair):
+    //   8 experts, k 2, D 512, I 256:    T = 128 (403 MB) 36, 46;   T = 512 (1.6 GB) 93, 72
+    //   16 experts, k 4, D 256, I 128:   T = 128 (201 MB) 32, 44;   T = 512 (805 MB) 73, 59
+    //   64 experts, k 8, D 512, I 256:   T = 24 (302 MB) 46, 49;    T = 40 (503 MB) 60, 54
+    //   256 experts, k 8, D 2048, I 512: T = 4 (403 MB) 81, 86; T = 8 144, 148 (with every token on
+    //   the same 8 experts 112, 59); T = 12 203, 197
     const bool kernels = f32_group_supported(D) && f32_group_supported(I) && (!S || S == I);
-    const bool group = kernels && 3 * P >= E && g.words <= (size_t)T * E;
+    const bool enough = (long long)P * D * I > 36000000;
+    // Rows per tile: 64 at most, fewer while the gate/up launch has under 8192 workgroups, which walk
+    // a tile's rows one after the other (8 experts, k 2, D = I = 1024, tiles of 8 / 16 / 64 rows: T = 64
+    // 68 / 73 / 81 us, 512 271 / 257 / 275, 2048 980 / 907 / 883); more where the grid would not
+    // hold them.
     constexpr int kPiece = 8;  // plain rows per workgroup
-    const int slots = group ? (E < P ? E : P) : P;
-    const bool fits = (T + kPiece - 1) / kPiece + slots <= kF32GroupMaxSlots;
-    if (kernels && fits && (group || P <= 4096)) {
+    const int pieces = (T + kPiece - 1) / kPiece, active = E < P ? E : P;
+    int tile_m = 8;
+    while (tile_m < 64 && (long long)(P / (2 * tile_m)) * f32_group_blocks(D, I, true) >= 8192) tile_m *= 2;
+    while (pieces + P / tile_m + active > kF32GroupMaxSlots && tile_m < P) tile_m *= 2;
+    const int max_tiles = P / tile_m + active;
+    struct {
+        size_t counts, offsets, order, tiles, n_tiles, words;
+    } g{};
+    g.offsets = permute_counts_words(P, E), g.order = g.offsets + E + 1, g.tiles = g.order + P;
+    g.n_tiles = g.tiles + 3 * (size_t)max_tiles, g.words = g.n_tiles + 1;
+    const bool group = enough && g.words <= (size_t)T * E;
+    const int slots = group ? max_tiles : P;
+    const bool fits = pieces + slots <= kF32GroupMaxSlots;
+    if (kernels && fits) {
         F32Group r{};
         r.K = D, r.N = E, r.pA = x, r.pW0 = W(m.gate.q), r.pout = logits, r.plain_rows = T, r.piece = kPiece;
         if (S) r.xW = W(m.shared_expert_gate.q), r.xout = sh_logit;
@@ -877,10 +891,10 @@ static Status sparse_moe_forward_f32(const mrun_sparse_moe &m, const float *x, i
         gu.ids = ids;
         if (group) {
             PermuteOut po{};
-            po.offsets = rt + g.offsets, po.order = rt + g.order, po.active = rt + g.active;
-            po.n_active = rt + g.n_active, po.tile_m = kGemmTileM;
+            po.offsets = rt + g.offsets, po.order = rt + g.order, po.tiles = rt + g.tiles;
+            po.n_tiles = rt + g.n_tiles, po.tile_m = tile_m;
             TRY_HIP(launch_permute(ids, P, k, E, rt + g.counts, po, s), "f32 permute");
-            gu.offsets = po.offsets, gu.order = po.order, gu.active = po.active, gu.n_active = po.n_active;
+            gu.order = po.order, gu.tiles = po.tiles, gu.n_tiles = po.n_tiles;
         }
         F32Group dn = gu;
         gu.K = D, gu.N = I, gu.A = x, gu.a_div = k, gu.out = act;
