@@ -11,6 +11,7 @@
 // Nothing here allocates device memory: scratch comes from the caller's workspace.
 #include <hip/hip_runtime.h>
 
+#include <climits>
 #include <cstdint>
 #include <cstring>
 #include <mutex>
@@ -310,16 +311,24 @@ static bool linear_q8(const mrun_linear &l) {
 }
 
 // Linear::forward (load.rs:294-306), dense or quantized. `zero` [n_zero] is cleared before the
-// product's results are visible to later launches (the prefill routing counters).
+// product's results are visible to later launches (the prefill routing counters). 8-bit weights run
+// the dense kernel for launches of up to max_blocks workgroups (of 64 x 64) or inputs of 4096 and more;
+// with more workgroups the generic GEMM fits more of them on a CU (us, generic and dense: 16384 rows x
+// 512, in 512 27 and 46, in 2048 97 and 124, in 4096 227 and 224; 4096 rows x 256, in 2048 25 and 17).
+// A block's router and gate take it at any size: a token's logits then have the same bits in every
+// prefill batch, and the block's one launch of both saves more (block of 256 experts, D 2048, generic
+// and dense: T = 6000 577 and 557 us, 12000 1024 and 1032, 24000 1974 and 2005).
+constexpr int kLinearMaxBlocks = 256;  // one per CU: a Linear on its own
 static Status linear(const bf16_t *x, int rows, const mrun_linear &l, bf16_t *y, hipStream_t s,
-                     uint32_t *zero = nullptr, int n_zero = 0) {
+                     uint32_t *zero = nullptr, int n_zero = 0, long long max_blocks = LLONG_MAX) {
     if (l.weight) {
         // the MFMA branches clear `zero` themselves
         const bool mfma = dense_gemm_supported(rows, l.in) || (rows > 16 && !(l.out < 16) && l.in % 64 == 0);
         if (zero && !mfma) TRY_HIP(launch_fill_u32(zero, 0u, n_zero, s), "clear");
         return linear_dense(x, rows, l, y, s, mfma ? zero : nullptr, n_zero);
     }
-    if (linear_q8(l) && dense_gemm_supported(rows, l.in)) {
+    const long long blocks = ((long long)rows + 63) / 64 * ((l.out + 63) / 64);
+    if (linear_q8(l) && dense_gemm_supported(rows, l.in) && (blocks <= max_blocks || l.in >= 4096)) {
         DenseJob j{};
         j.A = x, j.lda = l.in, j.M = rows, j.K = l.in;
         j.q0 = qw_of(l.q), j.bias0 = l.bias, j.N0 = l.out, j.out0 = y, j.ldo0 = l.out;
@@ -1294,7 +1303,8 @@ int mrun_linear_forward(const mrun_linear *l, const mrun_bf16 *x, int32_t rows, 
     if (st.ok() && rows == 0) return report(st);  // an empty batch: nothing to do
     if (st.ok()) st = check_ptr(x, "x");
     if (st.ok()) st = check_ptr(out, "out");
-    if (st.ok()) st = tensor::linear(x, rows, *l, out, (hipStream_t)stream);
+    if (st.ok())
+        st = tensor::linear(x, rows, *l, out, (hipStream_t)stream, nullptr, 0, tensor::kLinearMaxBlocks);
     return report(st);
 }
 
