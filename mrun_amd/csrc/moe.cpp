@@ -1250,7 +1250,15 @@ int mrun_gather_qmm(const mrun_bf16 *x, int32_t x_rows, const mrun_quantized *w,
             mj.glu = 0, mj.w0 = qw_of(*w), mj.routing = rt, mj.has_routing = 1;
             mj.max_tiles = (int)p.max_tiles, mj.out = (bf16_t *)(ws + p.ys), mj.ldo = w->out;
         }
-        const bool tuned = n > 16 && moe_gemm_supported(mj);
+        // The formats of moe_fmt.hip take it where the generic GEMM has enough to do (row tiles times 64
+        // columns times inputs; twice that with a single column block): the packing and the gather are
+        // two more launches, 6 us (us, generic and grouped, 8-bit group 64: 8 experts, in 1024, out 512,
+        // n = 64 23 and 29, in 2048, out 4096, n = 64 43 and 40, in 1024, out 1024, n = 4096 48 and 44;
+        // 128 experts, in 2048, out 256, n = 4096 40 and 46, out 1024, n = 17 52 and 38).
+        const bool fmt = w->bits != 4 || w->group_size != 64;
+        const size_t work = p.max_tiles * (size_t)(w->out / 64) * (size_t)w->in;
+        const bool pays = !fmt || work >= (w->out < 512 ? 1600000u : 800000u);
+        const bool tuned = n > 16 && pays && moe_gemm_supported(mj);
         if (tuned) po.inverse = u32(p.inverse), po.tile_rows = u32(p.tile_rows);
         st = hip_status(launch_permute(indices, n, tuned ? per_x : 1, E, u32(p.counts), po, s),
                         "gather_qmm permute");

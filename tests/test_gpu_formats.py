@@ -78,18 +78,19 @@ def test_mixed_formats(gate, down):
         run_block(hb, M.SparseMoe(hb), _x(hb.shape, T), f"gate/up {gate} down {down} T={T}")
 
 
-# 1024 inputs: the grouped GEMM (groups of 32 and bf16 weights: the generic one); 640: the generic one
-@pytest.mark.parametrize("hidden", [1024, 640])
+# 128 experts: enough work for the grouped GEMM (groups of 32 and bf16 weights: the generic one); with
+# 8, only group 64 takes it; 640 inputs: the generic one
+@pytest.mark.parametrize("hidden,experts", [(1024, 128), (1024, 8), (640, 8)])
 @pytest.mark.parametrize("bits,group", [(4, 64)] + FORMATS)
-def test_gather_qmm(bits, group, hidden):
+def test_gather_qmm(bits, group, hidden, experts):
     """gather_qmm above 16 indices in every format: unsorted indices, x rows shared by two."""
-    q = _host(bits, group, layer=6, hidden=hidden).gate_proj
+    q = _host(bits, group, layer=6, hidden=hidden, experts=experts).gate_proj
     n, rows = 150, 75
     ids = np.random.default_rng(1).integers(0, q.experts, n).astype(np.uint32)
     x = _x(synth.Shape(q.in_, 1, 1, 32), rows)
     got = M.bf16_bits(M.gather_qmm(M.bf16_tensor(x), M.DeviceQTensor(q), M.u32_tensor(ids)))
     ref = O.gather_qmm(q, x, ids)
-    assert_close(got, ref, what=f"gather_qmm {bits}-bit group {group} in {hidden}")
+    assert_close(got, ref, what=f"gather_qmm {bits}-bit group {group} in {hidden} experts {experts}")
 
 
 @pytest.mark.parametrize("T", [900, 1500, 2600, 6000])
