@@ -1,4 +1,4 @@
-// Decode schedule of the MoE block (T <= 16 tokens, T*k <= 128 pairs): three launches, no global
+// Decode schedule of the MoE block (T <= 32 tokens, T*k <= 256 pairs): three launches, no global
 // routing round trip and no permutation (SparseMoe::forward, moe.rs:149-174).
 //
 //   K1 router  : router logits (+ bias) and the shared expert's gate logit, one wave per row.

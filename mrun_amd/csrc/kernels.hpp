@@ -195,10 +195,11 @@ constexpr int kGemmTileN = 64;
 // 32 or 128, 8-bit and bf16 weights: moe_fmt.hip; biases may be null), K % 512 == 0, N a multiple
 // of 128 (glu) or 256. A is packed (launch_apack) with its X splits AX [rows][3][ax_e] (one entry
 // per ax_g inputs: 32 for weights in groups of 32, else 64; bf16 weights read none).
-// Routed tiles come from routing.tiles (64 rows); their A rows from tile_rows [tile][64] (token
-// of each tile row; only the tile's rows are read, rows past them repeat its last one) or,
-// without tile_rows, the sorted positions themselves. glu: out = packed R(silu(R(A.w0)) * R(A.w1)) and OX
-// [rows][3][N / ox_g] the X splits of each output row's groups of ox_g (0: none); else out = R(A.w0). The shared product (sh)
+// Routed tiles come from routing.tiles (of tile_m rows); their A rows from tile_rows [tile][tile_m]
+// (token of each tile row; only the tile's rows are read, rows past them repeat its last one) or,
+// without tile_rows, the sorted positions themselves. glu: out = packed R(silu(R(A.w0)) * R(A.w1)) and
+// OX [rows][3][N / ox_g] the X splits of each output row's groups of ox_g (0: none); else
+// out = R(A.w0). The shared product (sh)
 // has the same K and N and comes first.
 struct MoeGemmJob {
     const bf16_t *A;

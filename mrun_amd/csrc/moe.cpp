@@ -404,13 +404,16 @@ struct FusedNorm {
 // 2048 wide, that launch also takes the stack's residual add and next RMSNorm (post_done set, and
 // `out` is not written).
 // Prefill batches whose experts average at most this many rows have their routed tiles cut to 32
-// rows for the grouped GEMM. On the configs[1] block (per block, 32- against 64-row tiles):
+// rows for the grouped GEMM. On the Qwen3.6-like block (per block, 32- against 64-row tiles):
 // T = 33 131 -> 111 us, 64 154 -> 132, 128 164 -> 144, 256 180 -> 159, 512 190 -> 165, 768 199 ->
 // 179; T = 1024 (32 rows on average) the same; T = 2048 281 -> 308 (Zipf router: 268 -> 311).
 // 4-bit experts in groups of 32 or 128 (moe_fmt.hip), whose 32-row tiles run the longer ring, go on
-// to 32 rows: group 32 T = 900 (28.1 rows) 275 -> 233 us, T = 1200 (37.5 rows) 270 -> 280 (with the
-// even split of both), group 128 T = 900 192 -> 171, 1050 193 -> 191, 1200 197 -> 213. 8-bit experts
-// as group 64: T = 900 257 against 258, T = 1000 259 -> 271.
+// to 32 rows: us on 32- and 64-row tiles at 27, 30 and 34 rows, group 32: the same block 217 / 238,
+// 228 / 241, 242 / 246; 128 experts of 5120 x 1536 712 / 777, 754 / 772, 823 / 782; 512 of 1024 x 512
+// 196 / 209, 209 / 209, 233 / 213; 64 of 7168 x 2048 739 / 754, 801 / 760, 880 / 764 (16 of 4096 x 2048
+// only to 24 rows: 103 / 121, then 138 / 123, its few 64-row tiles being one per CU); group 128 the
+// same within 5 %. 8-bit experts as group 64: at 27 and 30 rows 241 / 250, 257 / 251, but 5120 x 1536
+// 866 / 808 and 7168 x 2048 773 / 701 already at 27.
 constexpr int kHalfTileMaxRows = 28, kHalfTileMaxRowsFmt4 = 32;
 
 // the largest batch that runs as decode-schedule chunks of at most 16 tokens, when the decode

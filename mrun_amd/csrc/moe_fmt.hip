@@ -12,9 +12,9 @@
 //  - A stage holds 64 or 128 bytes of each weight row: two K steps (of 64) of 4-bit codes, one of
 //    8-bit codes, or one of bf16 weights (whole 128-byte lines). Where a stage is at
 //    most 24 KB (8-bit codes, and 4-bit ones in 32-row tiles) the ring has three: the scales then
-//    go to registers, a chunk ahead, which frees their LDS (8-bit T = 1000 269.8 -> 262.0 us, group
-//    32 T = 700 241.6 -> 233.2). With two stages they stay in LDS (in registers, group 128 T = 1200
-//    took 197 us for 191).
+//    go to registers, a chunk ahead, which frees their LDS (block forward, 8-bit T = 1000 and group
+//    32 T = 700: 3 % faster than with two). With two stages they stay in LDS (in registers, group 128
+//    T = 1200 took 3 % longer).
 //  - 8-bit codes become exact bf16 integers (no offset); each dword holds codes i and i + 4 of a
 //    block, as the packed A has them. bf16 weights are re-paired the same way and go to the MFMAs
 //    without scales, straight into the accumulators.
@@ -24,9 +24,9 @@
 //  - Groups of 128: the two K steps of a group apply the same scale; the X sums stay per 64.
 //  - The LDS reads of a K step and their wait are one asm statement.
 // Measured on the Qwen3.6-like block, whole forwards, against the register-staged GEMM of qgemm.hip
-// (64 x 64 tiles, the shared expert in two launches of its own): 8-bit experts T = 1000 472 -> 265
-// us, 4-bit group 32 T = 700 545 -> 222, bf16 T = 300 676 -> 342 (1.6 GB of weights: 4.7 TB/s, near
-// the rate of a large copy).
+// (64 x 64 tiles, the shared expert in two launches of its own), both in turn: 8-bit experts T = 1000
+// 465 -> 262 us, 4-bit group 32 T = 700 540 -> 220, bf16 T = 300 677 -> 328 (1.6 GB of weights:
+// 4.9 TB/s, the rate of a large copy).
 #include <type_traits>
 
 #include "apack.hpp"
@@ -134,8 +134,11 @@ __global__ __launch_bounds__(256, 2) void fmt_gemm_kernel(MoeGemmJob j) {
     // on 64 workgroups: 46 with three each, not 8 with three and 56 with two), for the gate/up
     // products of bf16 weights and of groups of 32. Each workgroup streams whole lines of 256 weight
     // rows (and, for groups of 32, of their scales and biases, 16 bytes of a line at a time), so
-    // fewer of them keep those lines in the XCD's L2: bf16 T = 200 / 300 / 600 342 -> 322, 388 -> 351,
-    // 395 -> 364 us per block, group 32 T = 200 / 700 / 1600 207 -> 194, 221 -> 211, 302 -> 291. The
+    // fewer of them keep those lines in the XCD's L2. Block forwards, us, every workgroup against the
+    // even split: Qwen3.6-like, bf16 T = 256 345 -> 325, 768 353 -> 345, group 32 T = 256 209 -> 193,
+    // 768 220 -> 209; 128 experts of 2048 x 1024, bf16 T = 128 396 -> 356, group 32 T = 256 217 -> 206;
+    // 64 experts of 4096 x 1536, group 32 T = 256 327 -> 299 (but T = 341 343 -> 360, the worst of
+    // eight shapes); blocks with an item or less per workgroup the same. The
     // other formats need the loads in flight (8-bit T = 700 236 -> 247 us, group 128 157 -> 163), the
     // down products measured the same, and with more items the last round is a small part (group 32
     // T = 3000 423 -> 435, bf16 T = 2000 490 -> 492).

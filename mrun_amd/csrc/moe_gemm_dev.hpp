@@ -73,21 +73,11 @@ __device__ __forceinline__ uint32_t mg_neg128(uint32_t w) {
 // run on the VALU, and without this the compiler would treat their results (and the loads and
 // branches that depend on them) as per-lane.
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-// A pointer the whole wave holds, in scalar registers (so that a per-lane choice between two such
-// pointers is a select of values, not a per-lane load of the kernel argument holding them).
-template <class T>
-__device__ __forceinline__ const T *unip(const T *p) {
-    const uint64_t v = (uint64_t)(uintptr_t)p;
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return (const T *)(uintptr_t)(((uint64_t)hi << 32) | lo);
-}
 
 // LDS swizzles (16-byte units). A rows are 128 B (8 units): rows r and r + 8 (same bank window
 // at 256 B per cycle) and rows of one parity in 16 get distinct masks. B rows are 64 B (4 units,
-// two K steps of codes): the 4 rows of a 256-byte window... rows r, r + 4, r + 8, r + 12 (which
-// share a position in a 256-byte window) get distinct masks, and so do r, r + 2, r + 4, r + 6
-// (a 128-byte window).
+// two K steps of codes): rows r, r + 4, r + 8, r + 12 (which share a position in a 256-byte window)
+// get distinct masks, and so do r, r + 2, r + 4, r + 6 (a 128-byte window).
 __device__ __forceinline__ int swz_a(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 __device__ __forceinline__ int swz_c(int r) { return ((r >> 2) ^ (r >> 1)) & 3; }
 
@@ -100,7 +90,6 @@ __device__ __forceinline__ int xrow_of(int l) {
     return 32 * (fr >> 4) + 8 * ((fr >> 2) & 3) + 4 * (l >> 5) + (fr & 3);
 }
 
-
 // The gate/up epilogue of one wave's 32 NMI rows x 32 act columns (`col`: this lane's): act =
 // R(silu(R(gate)) * R(up)) of the fragments acc[.][0] (gate) and acc[.][1] (up), stored packed
 // through r_out (the tile's rows; stores past them are dropped). Returns the sum of the wave's 32
@@ -109,7 +98,7 @@ template <int NMI>
 __device__ __forceinline__ float store_act(const mg_f32x16 (&acc)[NMI][2], rsrc_t r_out, int ldo,
                                            int col, int lane) {
     const int fh = lane >> 5;
-        const int c64 = col & 63, kb = c64 >> 3, jj = c64 & 7;
+    const int c64 = col & 63, kb = c64 >> 3, jj = c64 & 7;
     // lanes with jj < 4 store packed pair (jj, jj + 4) of rows i (i even); lanes jj >= 4
     // the pair of row i + 1: both at the packed position of jj & 3
     const int pcol = (col & ~63) + 8 * (2 * (kb & 3) + (kb >> 2)) + 2 * (jj & 3);

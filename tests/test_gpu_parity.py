@@ -549,7 +549,7 @@ def q8_blocks():
 @pytest.mark.parametrize("T", [1, 3, 16, 24, 40, 300])
 def test_8bit_weights_match_oracle(q8_blocks, kind, T):
     """8-bit experts run the decode kernels at T <= 32 (each byte's two nibbles dotted as two 4-bit
-    codes; T = 24 as one batch of 192 pairs) and the generic MFMA GEMM above; an 8-bit router and
+    codes; T = 24 as one batch of 192 pairs) and the grouped MFMA GEMM above; an 8-bit router and
     shared gate are dequantized inside the decode router launch (T <= 32) or run as the prefill's
     first product."""
     hb, dev = q8_blocks[kind]
@@ -584,7 +584,7 @@ def test_8bit_groups(group):
 def test_groups_on_the_decode_kernels(group):
     """4-bit experts with groups of 32 and 128 on the Qwen3.6-like shape: the decode kernels (a
     lane's 32-code chunk lies in one group, its scale and bias picked by the group shift) at
-    T = 1, 4 and 24, and the generic MFMA GEMM at T = 300."""
+    T = 1, 4 and 24, and the grouped MFMA GEMM at T = 300."""
     shape = synth.Shape(hidden=2048, experts=256, top_k=8, intermediate=512, shared=512,
                         group=group)
     hb = synth.make_block(shape, config=synth.CFG_DECODE, layer=group)
@@ -650,7 +650,8 @@ def dense_block():
 
 @pytest.mark.parametrize("T", [1, 3, 16, 40, 300])
 def test_dense_experts_match_oracle(dense_block, T):
-    """Unquantized bf16 experts and shared expert (bits 16) on the generic GEMV and MFMA GEMM."""
+    """Unquantized bf16 experts and shared expert (bits 16) on the generic GEMV, and the grouped MFMA
+    GEMM from T = 40."""
     hb, dev = dense_block
     run_block(hb, dev, synth.make_x(Q8, T, config=synth.CFG_DECODE, layer=200 + T), f"dense T={T}")
 

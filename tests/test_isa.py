@@ -1,10 +1,12 @@
-"""Checks of the grouped GEMM's machine code (CPU only: hipcc cross-compiles for gfx950).
+"""Checks of the grouped GEMMs' machine code (CPU only: hipcc cross-compiles for gfx950).
 
-The grouped GEMM issues its LDS reads as inline asm and waits for them with separate lgkmcnt
+The group-64 GEMM issues its LDS reads as inline asm and waits for them with separate lgkmcnt
 statements, so the compiler takes a destination register as written at issue. A spill, copy or
 other use of that register before the wait that covers the read would see a value the load has not
 yet filled. These tests compile the kernel the way the library is built and check its assembly:
-no VGPR spills or scratch, and no instruction touching a pending destination register.
+no VGPR spills or scratch, and no instruction touching a pending destination register. The GEMM of
+the other formats waits in the statement that reads, so there a spill would only cost time; its
+widest instantiations sit at the register limit, and are checked for spills too.
 """
 import re
 import shutil
@@ -31,13 +33,17 @@ def _regs(text):
     return out
 
 
-@pytest.fixture(scope="module")
-def gemm_asm(tmp_path_factory):
-    out = tmp_path_factory.mktemp("isa") / "moe_gemm.s"
+def _asm(tmp_path_factory, name):
+    out = tmp_path_factory.mktemp("isa") / f"{name}.s"
     flags = [f for f in B.HIP_FLAGS if f != "-fPIC"]
-    subprocess.run([B.HIPCC, *flags, "--cuda-device-only", "-S", str(B.CSRC / "moe_gemm.hip"), "-o",
+    subprocess.run([B.HIPCC, *flags, "--cuda-device-only", "-S", str(B.CSRC / f"{name}.hip"), "-o",
                     str(out)], check=True, capture_output=True)
     return out.read_text()
+
+
+@pytest.fixture(scope="module")
+def gemm_asm(tmp_path_factory):
+    return _asm(tmp_path_factory, "moe_gemm")
 
 
 def _kernel_bodies(asm):
@@ -50,13 +56,28 @@ def _kernel_bodies(asm):
     return bodies
 
 
+def _assert_no_spills(asm, name, body):
+    desc = asm[asm.index(f".amdhsa_kernel {name}"):]
+    desc = desc[:desc.index(".end_amdhsa_kernel")]
+    m = re.search(r"\.amdhsa_private_segment_fixed_size\s+(\d+)", desc)
+    assert m is not None and int(m.group(1)) == 0, f"{name} uses scratch"
+    assert not any("scratch_" in ln for ln in body), f"{name} spills VGPRs"
+
+
 def test_grouped_gemm_has_no_spills(gemm_asm):
     for name, body in _kernel_bodies(gemm_asm).items():
-        desc = gemm_asm[gemm_asm.index(f".amdhsa_kernel {name}"):]
-        desc = desc[:desc.index(".end_amdhsa_kernel")]
-        m = re.search(r"\.amdhsa_private_segment_fixed_size\s+(\d+)", desc)
-        assert m is not None and int(m.group(1)) == 0, f"{name} uses scratch"
-        assert not any("scratch_" in ln for ln in body), f"{name} spills VGPRs"
+        _assert_no_spills(gemm_asm, name, body)
+
+
+def test_format_gemm_has_no_spills(tmp_path_factory):
+    asm = _asm(tmp_path_factory, "moe_fmt")
+    names = re.findall(r"^(_ZN4mrun15fmt_gemm_kernelI\w+):", asm, re.M)
+    # gate/up and down of 8-bit groups of 32, 64, 128 and 4-bit ones of 32, 128 in both tile heights,
+    # and of bf16 weights in 32-row tiles
+    assert len(names) == 22
+    for name in names:
+        start = asm.index(f"\n{name}:") + 1
+        _assert_no_spills(asm, name, asm[start:asm.index("s_endpgm", start)].splitlines())
 
 
 def test_asm_lds_reads_are_not_touched_before_their_wait(gemm_asm):
